@@ -180,9 +180,9 @@ def _inputs(c, seed):
         dt = torch.float32 if c["x"] == "f32" else torch.bfloat16
         s["x"] = torch.randn((c["layers"], c["m"], c["k"]), device=DEV, generator=g).to(dt)
         if c["epilogue"] == "bias":
-            s["bias"] = torch.randn((c["layers"], c["n"]), device=DEV, generator=g)
+            s["bias"] = [torch.randn(c["n"], device=DEV, generator=g) for _ in range(c["layers"])]
         if c["epilogue"] == "residual":
-            s["residual"] = torch.randn((c["layers"], c["m"], c["n"]), device=DEV, generator=g)
+            s["residual"] = [torch.randn((c["m"], c["n"]), device=DEV, generator=g) for _ in range(c["layers"])]
     elif c["kind"] == "moe":
         s["logits"] = [_logits(c, g) for _ in range(c["layers"])]
         s["x"] = torch.randn((c["layers"], c["t"], c["dm"]), device=DEV, generator=g).to(torch.bfloat16)
@@ -207,8 +207,8 @@ def prepare(case, seed):
         rows = c["n"] * (2 if c["epilogue"] == "swiglu" else 1)
         s["w"] = [_device_weight(c["scheme"], rows, c["k"], _weight_gen(seed, i)) for i in range(c["layers"])]
         if c["graph"]:
-            s["y"] = torch.empty((c["layers"], c["m"], c["n"]), device=DEV,
-                                 dtype=torch.float32 if c["out"] == "f32" else torch.bfloat16)
+            s["y"] = [torch.empty((c["m"], c["n"]), device=DEV, dtype=torch.float32 if c["out"] == "f32"
+                                  else torch.bfloat16) for _ in range(c["layers"])]
     else:
         n = c.get("layers", 1)
         s["ids"] = torch.empty((n, c["t"], c["top_k"]), dtype=torch.int32, device=DEV)
@@ -236,15 +236,12 @@ def prepare(case, seed):
 def _pass(s):
     c = s["case"]
     if c["kind"] == "matmul":
-        ys = []
-        for i, (w, scales) in enumerate(s["w"]):
-            ys.append(ffi.matmul(w, SCHEMES[c["scheme"]], c["n"], c["k"], s["x"][i],
-                                 out_dtype=ffi.F32 if c["out"] == "f32" else ffi.BF16,
-                                 bias=s["bias"][i] if "bias" in s else None,
-                                 residual=s["residual"][i] if "residual" in s else None,
-                                 y=s["y"][i] if "y" in s else None, w_scales=scales,
-                                 swiglu=c["epilogue"] == "swiglu"))
-        return s["y"] if "y" in s else ys
+        return [ffi.matmul(w, SCHEMES[c["scheme"]], c["n"], c["k"], s["x"][i],
+                           out_dtype=ffi.F32 if c["out"] == "f32" else ffi.BF16,
+                           bias=s["bias"][i] if "bias" in s else None,
+                           residual=s["residual"][i] if "residual" in s else None,
+                           y=s["y"][i] if "y" in s else None, w_scales=scales, swiglu=c["epilogue"] == "swiglu")
+                for i, (w, scales) in enumerate(s["w"])]
     for i, logits in enumerate(s["logits"]):
         ids, weights = ffi.moe_route(logits, c["top_k"], scoring=ffi.SCORING_SIGMOID if c.get("scoring") == "sigmoid"
                                      else ffi.SCORING_SOFTMAX, ids=s["ids"][i], weights=s["weights"][i],
@@ -375,7 +372,7 @@ def exact(case, seed):
                 y = torch.nn.functional.silu(y[:, :c["n"]]) * y[:, c["n"]:]
             y = y + s["bias"][i] if "bias" in s else y + s["residual"][i] if "residual" in s else y
             ys.append(y)
-        return torch.stack(ys) if c["graph"] else ys
+        return ys
     routed = [_exact_route(z, c["top_k"], c.get("scoring") == "sigmoid") for z in s["logits"]]
     out = {"ids": None, "weights": torch.stack([w for _, w in routed])}
     if c["kind"] == "route":
