@@ -7,7 +7,8 @@
  * T0 meaning: crates/r9v-t0/src/matmul.rs:1940-2414 (Branch D), output cast
  * crates/r9v-t0/src/dtype.rs:102-111 (bf16 RNE); epilogue matmul.rs:2421-2446.
  *
- * Two launches:
+ * Launches whose rows do not fill these tiles go to the thin tiles of
+ * gemm_thin.hip (thin_plan, below).  Two launches:
  *  1. x_to_f16: one wave per activation row finds max|x|, picks the
  *     power-of-two scale 2^e that keeps the row below 2^15 (e = 0 for any
  *     ordinary activation) and writes the row as fp16 plus the scale, in the
@@ -251,6 +252,34 @@ uint32_t plan_chunks(GemmArgs &a, uint32_t cus) {
     return (uint32_t)q;
 }
 
+/* Which kernel: both run in rounds of one workgroup per CU, and a workgroup's
+ * time per super-block (256 K) is a constant of its shape, so the launch with
+ * the least rounds x time is taken.  The constants are nanoseconds measured
+ * on Q4_K at k = 4096 (launch times less 8 us, over 16 super-blocks; the other
+ * schemes' are within 20% in the same order).  A 256-column workgroup's step
+ * costs 2900 whatever its rows and 680 per row tile; the thin tiles' cost
+ * follows their shape.  k = 4096, us, 256-column tiles / the chosen thin ones:
+ *   n = 4096:  m = 32: 61 / 16, 128: 60 / 20, 512: 62 / 36, 1024: 71 / 64
+ *   n = 14336: m = 32: 62 / 25, 128: 63 / 32, 256: 71 / 56, 512: 99 / (107)
+ * and Q6_K n = 2048, k = 14336, m = 64: 254 / 44. */
+uint64_t gemm3_cost(const GemmArgs &a, uint32_t wgs, uint32_t cus) {
+    const uint32_t per = (a.rt + a.nlo - 1) / a.nlo; /* row tiles of the largest chunk */
+    return (uint64_t)((wgs + cus - 1) / cus) * (2900u + 680u * per);
+}
+
+uint64_t thin_plan(uint32_t m, uint32_t n, uint32_t cus, uint32_t &nr, uint32_t &nc) {
+    static const struct {
+        uint32_t nr, nc, ns;
+    } kShapes[] = {{1, 1, 500}, {2, 1, 600}, {4, 1, 900}, {1, 2, 930}, {2, 2, 1060}, {4, 2, 1400}};
+    uint64_t best = ~0ull;
+    for (const auto &s : kShapes) {
+        const uint64_t wgs = (uint64_t)((n + 32 * s.nc - 1) / (32 * s.nc)) * ((m + 32 * s.nr - 1) / (32 * s.nr));
+        const uint64_t cost = (wgs + cus - 1) / cus * s.ns;
+        if (cost < best) best = cost, nr = s.nr, nc = s.nc;
+    }
+    return best;
+}
+
 }  // namespace
 
 uint32_t r9vx_device_cus() {
@@ -265,8 +294,10 @@ uint32_t r9vx_device_cus() {
     return cached[dev];
 }
 
+size_t r9vx_gemm_x16_bytes(uint32_t m, uint32_t k) { return (size_t)((m + 31) & ~31u) * k * 2; }
+
 size_t r9vx_gemm_workspace_bytes(uint32_t m_bucket, uint32_t k) {
-    return (((size_t)m_bucket * k * 2 + 255) & ~(size_t)255) + (size_t)m_bucket * 4;
+    return r9vx_gemm_x16_bytes(m_bucket, k) + (size_t)m_bucket * 4;
 }
 
 int r9vx_launch_x_to_f16(const uint16_t *x, uint32_t m, uint32_t k, _Float16 *x16, float *scale,
@@ -284,8 +315,7 @@ int r9vx_launch_x_to_f16(const uint16_t *x, uint32_t m, uint32_t k, _Float16 *x1
 
 int r9vx_launch_gemm(const r9vx_gemm_problem &p, hipStream_t stream) {
     _Float16 *x16 = reinterpret_cast<_Float16 *>(p.workspace);
-    float *scale = reinterpret_cast<float *>(reinterpret_cast<uint8_t *>(p.workspace) +
-                                             (((size_t)p.m * p.k * 2 + 255) & ~(size_t)255));
+    float *scale = reinterpret_cast<float *>(reinterpret_cast<uint8_t *>(p.workspace) + r9vx_gemm_x16_bytes(p.m, p.k));
     GemmArgs a{};
     a.x16 = x16;
     a.scale = scale;
@@ -306,18 +336,24 @@ int r9vx_launch_gemm(const r9vx_gemm_problem &p, hipStream_t stream) {
     a.k = p.k;
     a.y_bf16 = p.y_dtype == R9VX_DTYPE_BF16;
     a.epilogue = p.epilogue;
-    /* One kernel for every scheme and shape (gemm3_kernel: 256 x 256 tiles,
-     * each weight tile decoded once into LDS), so each output element's
-     * arithmetic -- the K order of the MFMA steps, how a weight is rounded
-     * to fp16 -- follows from the scheme and k alone, never from the
-     * launch's row count: a row's outputs are the same bits whatever rows
-     * share the launch, at whatever index, and in every bucket above the
-     * decode GEMV's.  The A copies address x16 with 32-bit offsets, so rows
-     * go in launches of at most 2^31 / k elements' worth (which rows share a
-     * launch changes no bit either). */
+    /* Two kernels for every scheme and shape, chosen by size: gemm3_kernel
+     * (256 x 256 tiles) and the thin tiles of gemm_thin.hip.  Both give each
+     * output element the same arithmetic -- the K order of the MFMA slices,
+     * how a weight is rounded to fp16 -- which follows from the scheme and k
+     * alone, never from the launch's row count: a row's outputs are the same
+     * bits whatever rows share the launch, at whatever index, and in every
+     * bucket above the decode GEMV's.  The A copies address x16 with 32-bit
+     * offsets, so rows go in launches of at most 2^31 / k elements' worth
+     * (which rows share a launch changes no bit either). */
+    const uint32_t cus = r9vx_device_cus();
+    {
+        GemmArgs whole = a;
+        const uint32_t wgs = plan_chunks(whole, cus);
+        uint32_t nr = 0, nc = 0;
+        if (thin_plan(p.m, p.n, cus, nr, nc) < gemm3_cost(whole, wgs, cus)) return r9vx_launch_gemm_thin(p, nr, nc, stream);
+    }
     const int rc = r9vx_launch_x_to_f16(p.x, p.m, p.k, x16, scale, r9vx_group_order(p.scheme), stream);
     if (rc) return rc;
-    const uint32_t cus = r9vx_device_cus();
     const uint32_t max_rows = (uint32_t)(((1ull << 31) - 1) / p.k) & ~31u;
     const size_t ysz = a.y_bf16 ? 2 : 4;
     for (uint32_t r0 = 0; r0 < p.m; r0 += max_rows) {

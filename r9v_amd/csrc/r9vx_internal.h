@@ -113,7 +113,12 @@ struct r9vx_gemm_problem {
     uint32_t scheme, y_dtype, epilogue;
 };
 size_t r9vx_gemm_workspace_bytes(uint32_t m_bucket, uint32_t k);
+/* Bytes of the fp16 rows in it, whole 32-row tiles; the row scales follow. */
+size_t r9vx_gemm_x16_bytes(uint32_t m, uint32_t k);
 int r9vx_launch_gemm(const r9vx_gemm_problem &p, hipStream_t stream);
+/* The thin-tile form (gemm_thin.hip): nr row tiles of 32 rows and nc column
+ * tiles of 32 columns per workgroup.  Output bits equal r9vx_launch_gemm's. */
+int r9vx_launch_gemm_thin(const r9vx_gemm_problem &p, uint32_t nr, uint32_t nc, hipStream_t stream);
 /* Compute units of the current device (cached per device; 256 if the query fails). */
 uint32_t r9vx_device_cus();
 
