@@ -136,11 +136,13 @@ __device__ void put_tile_lists(const SortArgs &a, uint32_t tot, uint32_t off, ui
     if (tid == 0) reinterpret_cast<uint32_t *>(a.ws + L.status)[4] = all3 + a.shared * s3;
 }
 
-/* P <= 1024 pairs: everything in one workgroup of 1024 threads. */
+/* P <= 1024 pairs: everything in one workgroup of 1024 threads (workgroup 0;
+ * the others convert activation rows). */
 __global__ __launch_bounds__(1024) void sort_small_kernel(SortArgs a) {
     __shared__ uint16_t cnt[16][kMoeMaxE];
     __shared__ uint32_t sh[16];
     __shared__ uint32_t bad_sh;
+    if (sort_x16_part(a, 1, 0, a.t)) return;
     const MoeLayout &L = a.L;
     uint32_t tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     for (uint32_t i = tid; i < 16 * kMoeMaxE; i += blockDim.x) (&cnt[0][0])[i] = 0;
@@ -1101,9 +1103,18 @@ static uint32_t lpr_for(uint32_t k, uint32_t &nseg) {
 
 int r9vx_moe_sort_stage(const r9vx_moe_problem &p, const MoeLayout &L, hipStream_t s, bool *x16_done) {
     SortArgs a{p.ids, p.ws, L, p.t * p.k, p.e, p.k, p.t, p.shared};
-    if (x16_done) *x16_done = false;
+    if (x16_done) {
+        a.x = p.x;
+        a.x16 = reinterpret_cast<_Float16 *>(p.ws + L.x16);
+        a.xscale = reinterpret_cast<float *>(p.ws + L.xscale);
+        a.dm = p.dm;
+        a.xperm = r9vx_group_order(p.scheme_gu);
+        *x16_done = true;
+    }
     if (a.p <= 1024) {
-        hipLaunchKernelGGL(sort_small_kernel, dim3(1), dim3(1024), 0, s, a);
+        /* sixteen activation rows per further workgroup, beside the sort (a
+         * launch of their own took 5.3 us at T = 48) */
+        hipLaunchKernelGGL(sort_small_kernel, dim3(1 + (x16_done ? (a.t + 15) / 16 : 0)), dim3(1024), 0, s, a);
         return (int)hipGetLastError();
     }
     const uint32_t nchunk = (a.p + 255) / 256;
@@ -1113,14 +1124,8 @@ int r9vx_moe_sort_stage(const r9vx_moe_problem &p, const MoeLayout &L, hipStream
      * idle), four rows per 256-thread workgroup, sixteen per 1024 */
     uint32_t xr[5] = {0, 0, 0, 0, 0};
     if (x16_done) {
-        a.x = p.x;
-        a.x16 = reinterpret_cast<_Float16 *>(p.ws + L.x16);
-        a.xscale = reinterpret_cast<float *>(p.ws + L.xscale);
-        a.dm = p.dm;
-        a.xperm = r9vx_group_order(p.scheme_gu);
         constexpr uint32_t kCum[5] = {0, 20, 40, 80, 100};
         for (int i = 1; i <= 4; ++i) xr[i] = (uint32_t)((uint64_t)p.t * kCum[i] / 100);
-        *x16_done = true;
     }
     auto xblocks = [&](int i, uint32_t rows_per_block) { return (xr[i + 1] - xr[i] + rows_per_block - 1) / rows_per_block; };
     hipLaunchKernelGGL(sort_count_kernel, dim3(nchunk + xblocks(0, 4)), dim3(256), 0, s, a, xr[0], xr[1]);

@@ -103,7 +103,7 @@ struct MoeCombineArgs {
 inline bool r9vx_moe_decode_form(const r9vx_moe_problem &p) { return p.t_bucket <= 8; }
 
 /* x16_done != NULL: the sort kernels also convert the activation rows for
- * the grouped GEMMs (only on the multi-kernel path; *x16_done says whether). */
+ * the grouped GEMMs (*x16_done says so). */
 int r9vx_moe_sort_stage(const r9vx_moe_problem &p, const MoeLayout &L, hipStream_t s, bool *x16_done = nullptr);
 int r9vx_moe_decode_stage(const r9vx_moe_problem &p, const MoeLayout &L, hipStream_t s);
 int r9vx_moe_grouped_stage(const r9vx_moe_problem &p, const MoeLayout &L, hipStream_t s, bool x16_done = false);

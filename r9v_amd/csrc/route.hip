@@ -363,15 +363,28 @@ __global__ __launch_bounds__(256) void route_kernel(RouteArgs a) {
  * talking to each other; workgroup 0 writes the status word. */
 constexpr uint32_t kRouteSmallT = 8;
 
-template <int PER>
+/* More rows, up to kRouteMidT: the same with six checking waves, each taking
+ * its rows four at a time.  Reading T rows in T workgroups is L2 traffic that
+ * passes under the routing waves' chain at these sizes, where a check launch
+ * of its own (after one that clears the status word) does not: T = 48, E = 512,
+ * K = 10 11.2 us in three launches, 5.9 in one. */
+constexpr uint32_t kRouteMidT = 128;
+/* and up to this many logits, past which the workgroups' reads cost more than
+ * the launches: E = 512 T = 96 11.4 -> 8.7 us, T = 128 11.5 / 11.0; E = 1024
+ * T = 48 16.5 -> 10.1, T = 96 16.7 / 17.2; E = 64 T = 128 7.2 -> 5.2 */
+constexpr uint32_t kRouteMidLogits = 48u << 10;
+constexpr uint32_t kRouteCheckRows = 4; /* rows a checking wave loads at once */
+
+/* Rows first, first + STRIDE, ...: R of them. */
+template <int PER, int STRIDE>
 struct CheckRows {
-    static constexpr int R = kRouteSmallT / 2;
+    static constexpr int R = kRouteCheckRows;
     float lg[R][PER], bs[PER];
-    /* rows first, first + 2, ... (< T) and the bias: loads only */
+    /* rows first, first + STRIDE, ... (< T) and the bias: loads only */
     __device__ __forceinline__ void load(const RouteArgs &a, uint32_t first, uint32_t lane) {
 #pragma unroll
         for (int j = 0; j < R; ++j) {
-            const uint32_t r = first + 2 * j < a.t ? first + 2 * j : 0u; /* rows past T: row 0, unused */
+            const uint32_t r = first + STRIDE * j < a.t ? first + STRIDE * j : 0u; /* rows past T: row 0, unused */
 #pragma unroll
             for (int i = 0; i < PER; ++i) {
                 const uint32_t c = lane + 64 * i;
@@ -390,7 +403,7 @@ struct CheckRows {
         uint32_t bad = 0;
 #pragma unroll
         for (int j = 0; j < R; ++j) {
-            if (first + 2 * j >= a.t) break;
+            if (first + STRIDE * j >= a.t) break;
             float sc[PER], l[PER], b[PER];
 #pragma unroll
             for (int i = 0; i < PER; ++i) {
@@ -407,8 +420,11 @@ struct CheckRows {
     }
 };
 
-template <int PER>
-__global__ __launch_bounds__(256) void route_small_kernel(RouteArgs a) {
+/* CHECK: the checking waves (2: T <= kRouteSmallT, their rows loaded before the
+ * first barrier; 6: T <= kRouteMidT). */
+template <int PER, int CHECK>
+__global__ __launch_bounds__(64 * (2 + CHECK)) void route_small_kernel(RouteArgs a) {
+    static_assert(2 * kRouteCheckRows >= kRouteSmallT, "two waves hold every row");
     __shared__ uint32_t bad_all;
     __shared__ uint64_t etab[R9VX_EXP2F_N];
     __shared__ __attribute__((aligned(16))) float sbuf[PER * 64];
@@ -417,14 +433,19 @@ __global__ __launch_bounds__(256) void route_small_kernel(RouteArgs a) {
     r9vx_exp2_fill(etab, threadIdx.x, blockDim.x);
     if (threadIdx.x == 0) bad_all = 0;
     float sc[PER], lg[PER], bs[PER];
-    CheckRows<PER> cr;
+    CheckRows<PER, CHECK> cr;
     if (role < 2)
         load_row<PER>(a, row, lane, sc, lg, bs);
     else
         cr.load(a, role - 2, lane);
     __syncthreads();
     if (role >= 2) { /* the checking waves */
-        const uint32_t bad = cr.check(a, role - 2, lane, etab);
+        uint32_t bad = cr.check(a, role - 2, lane, etab);
+        if constexpr (CHECK > 2)
+            for (uint32_t first = role - 2 + CHECK * kRouteCheckRows; first < a.t; first += CHECK * kRouteCheckRows) {
+                cr.load(a, first, lane);
+                bad |= cr.check(a, first, lane, etab);
+            }
         if (bad && lane == 0) atomicOr(&bad_all, bad);
         __syncthreads();
         return;
@@ -650,7 +671,11 @@ int r9vx_launch_route_hidden(const r9vx_route_hidden_problem &p, hipStream_t str
 template <int PER>
 static int launch_route_per(const RouteArgs &a, hipStream_t stream) {
     if (a.t <= kRouteSmallT) {
-        hipLaunchKernelGGL((route_small_kernel<PER>), dim3(a.t), dim3(256), 0, stream, a);
+        hipLaunchKernelGGL((route_small_kernel<PER, 2>), dim3(a.t), dim3(256), 0, stream, a);
+        return (int)hipGetLastError();
+    }
+    if (a.t <= kRouteMidT && a.t * a.e <= kRouteMidLogits) {
+        hipLaunchKernelGGL((route_small_kernel<PER, 6>), dim3(a.t), dim3(512), 0, stream, a);
         return (int)hipGetLastError();
     }
     hipLaunchKernelGGL(clear_status_kernel, dim3(1), dim3(1), 0, stream, a.status);
