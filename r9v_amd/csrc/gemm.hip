@@ -294,7 +294,7 @@ uint32_t r9vx_device_cus() {
     return cached[dev];
 }
 
-size_t r9vx_gemm_x16_bytes(uint32_t m, uint32_t k) { return (size_t)((m + 31) & ~31u) * k * 2; }
+size_t r9vx_gemm_x16_bytes(uint32_t m, uint32_t k) { return ((size_t)m * k * 2 + 255) & ~(size_t)255; }
 
 size_t r9vx_gemm_workspace_bytes(uint32_t m_bucket, uint32_t k) {
     return r9vx_gemm_x16_bytes(m_bucket, k) + (size_t)m_bucket * 4;

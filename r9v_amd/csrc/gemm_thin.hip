@@ -51,8 +51,9 @@ struct ThinArgs {
  * bucket of 32 rows on 8 CUs: 6.7 -> 4.5 us at k = 4096): its max picks the power-of-two scale
  * (row_shift), and the row is written as fp16 in the weight scheme's K order,
  * so that an MFMA operand is one contiguous load: 32-row tile t's 8-element
- * group c / 8 of row r is at x16 + 32 t k + ((c / 8) 32 + r) 8 (rows past m
- * are not written).  The bits are those of x16_row.  K <= 8192 stays in registers
+ * group c / 8 of row r is at x16 + 32 t k + ((c / 8) R + r) 8, R the tile's
+ * rows (32, or what m leaves in the last: whole tiles there would take up to
+ * 31 rows more of the workspace than the rows themselves).  The bits are those of x16_row.  K <= 8192 stays in registers
  * between the max and the conversion. */
 template <int PERM>
 __global__ __launch_bounds__(256) void x_to_f16_thin_kernel(const uint16_t *__restrict__ x, uint32_t m, uint32_t k,
@@ -100,12 +101,13 @@ __global__ __launch_bounds__(256) void x_to_f16_thin_kernel(const uint16_t *__re
     const float inv = ldexpf(1.0f, -e);
     if (tid == 0) scale[row] = ldexpf(1.0f, e);
     _Float16 *const out = x16 + (uint64_t)(row & ~31u) * k + 8 * (row & 31u);
+    const uint32_t tile = row & ~31u, rows = m - tile < 32 ? m - tile : 32;
     auto put = [&](uint32_t c, const uint32_t (&v)[4]) {
         uint32_t o[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j)
             o[j] = pack_h2(__builtin_bit_cast(float, v[j] << 16) * inv, __builtin_bit_cast(float, v[j] & 0xFFFF0000u) * inv);
-        *reinterpret_cast<r9vx_u32x4 *>(out + 32ull * c) = r9vx_u32x4{o[0], o[1], o[2], o[3]};
+        *reinterpret_cast<r9vx_u32x4 *>(out + (uint64_t)rows * c) = r9vx_u32x4{o[0], o[1], o[2], o[3]};
     };
     if (hold) {
 #pragma unroll
@@ -206,16 +208,18 @@ __global__ __launch_bounds__(64 * (NR + kThinDec)) void gemm_thin_kernel(ThinArg
         for (uint32_t c = 0; c < nb; ++c) lds_barrier();
         return;
     }
-    /* rows past m in the last tile are whatever the workspace holds: a row's
-     * products stay in its own lane, which stores nothing */
-    const uint32_t nk = a.k / 64, aoff = (4 * h * 32 + (lane & 31)) * 16;
+    /* lanes past the last tile's rows read its last row again and store nothing */
+    const uint32_t nk = a.k / 64, ar = (lane & 31) < rows ? (lane & 31) : rows - 1;
+    uint32_t aoff[4]; /* slice s: group 4 h + s of a step's eight */
+#pragma unroll
+    for (int s = 0; s < 4; ++s) aoff[s] = ((4 * h + s) * rows + ar) * 16;
     const uint8_t *const abase = reinterpret_cast<const uint8_t *>(a.x16 + (uint64_t)32 * mt * a.k);
     /* A operands, five steps ahead: x16 comes from the L2 or, on an XCD's
      * first touch, from the memory side cache, hundreds of nanoseconds away */
     constexpr int kARing = thin_a_ring(NC);
     half8 af[kARing][4];
     auto load_a = [&](uint32_t step, int s, half8 &f) {
-        f = thin_ld<half8>(abase + (uint64_t)(step < nk ? step : nk - 1) * 4096u, aoff, 512 * s);
+        f = thin_ld<half8>(abase + (uint64_t)(step < nk ? step : nk - 1) * (128u * rows), aoff[s], 0);
     };
     r9vx_f32x16 acc[NC];
 #pragma unroll

@@ -113,7 +113,7 @@ struct r9vx_gemm_problem {
     uint32_t scheme, y_dtype, epilogue;
 };
 size_t r9vx_gemm_workspace_bytes(uint32_t m_bucket, uint32_t k);
-/* Bytes of the fp16 rows in it, whole 32-row tiles; the row scales follow. */
+/* Bytes of the fp16 rows in it; the row scales follow. */
 size_t r9vx_gemm_x16_bytes(uint32_t m, uint32_t k);
 int r9vx_launch_gemm(const r9vx_gemm_problem &p, hipStream_t stream);
 /* The thin-tile form (gemm_thin.hip): nr row tiles of 32 rows and nc column
