@@ -253,28 +253,51 @@ uint32_t plan_chunks(GemmArgs &a, uint32_t cus) {
 }
 
 /* Which kernel: both run in rounds of one workgroup per CU, and a workgroup's
- * time per super-block (256 K) is a constant of its shape, so the launch with
- * the least rounds x time is taken.  The constants are nanoseconds measured
+ * time per super-block (256 K) follows from its shape, so the launch with the
+ * least sum over its rounds is taken.  The constants are nanoseconds measured
  * on Q4_K at k = 4096 (launch times less 8 us, over 16 super-blocks; the other
  * schemes' are within 20% in the same order).  A 256-column workgroup's step
- * costs 2900 whatever its rows and 680 per row tile; the thin tiles' cost
- * follows their shape.  k = 4096, us, 256-column tiles / the chosen thin ones:
- *   n = 4096:  m = 32: 61 / 16, 128: 60 / 20, 512: 62 / 36, 1024: 71 / 64
- *   n = 14336: m = 32: 62 / 25, 128: 63 / 32, 256: 71 / 56, 512: 99 / (107)
- * and Q6_K n = 2048, k = 14336, m = 64: 254 / 44. */
+ * costs 2900 whatever its rows and 680 per row tile.  A thin one's follows its
+ * active row tiles and, where those read enough activations to fill the L2's
+ * bandwidth, how many of the CUs work beside it: 64 columns x 8 row tiles
+ * 2100 on 160 CUs, 2850 on 256.  k = 4096, us, 256-column tiles / thin ones:
+ *   n = 4096:  m = 32: 61 / 16, 128: 60 / 20, 512: 62 / 36, 1024: 71 / 54
+ *   n = 14336: m = 32: 62 / 25, 128: 63 / 32, 256: 71 / 48, 512: 104 / 85
+ * and Q6_K n = 2048, k = 14336, m = 64: 254 / 44.  Up to 4 row tiles a
+ * workgroup alone: n = 4096 m = 777 55 us (with 8: 48), 1024 65 (54). */
 uint64_t gemm3_cost(const GemmArgs &a, uint32_t wgs, uint32_t cus) {
     const uint32_t per = (a.rt + a.nlo - 1) / a.nlo; /* row tiles of the largest chunk */
     return (uint64_t)((wgs + cus - 1) / cus) * (2900u + 680u * per);
 }
 
+struct ThinShape {
+    uint32_t nr, nc, ns, load; /* ns + load x (the share of the CUs at work) */
+};
+constexpr ThinShape kThinShapes[] = {{1, 1, 500, 0},   {2, 1, 600, 0},    {4, 1, 900, 0},    {1, 2, 930, 0},
+                                     {2, 2, 1060, 0}, {4, 2, 900, 830}, {8, 2, 1300, 1500}};
+
+/* One round of `wgs` workgroups of nc column tiles and `tiles` active row tiles. */
+uint64_t thin_round(uint32_t nc, uint32_t tiles, uint64_t wgs, uint32_t cus) {
+    for (const auto &s : kThinShapes)
+        if (s.nc == nc && s.nr >= tiles) return s.ns + s.load * (wgs < cus ? wgs : cus) / cus;
+    return ~0u;
+}
+
 uint64_t thin_plan(uint32_t m, uint32_t n, uint32_t cus, uint32_t &nr, uint32_t &nc) {
-    static const struct {
-        uint32_t nr, nc, ns;
-    } kShapes[] = {{1, 1, 500}, {2, 1, 600}, {4, 1, 900}, {1, 2, 930}, {2, 2, 1060}, {4, 2, 1400}};
     uint64_t best = ~0ull;
-    for (const auto &s : kShapes) {
-        const uint64_t wgs = (uint64_t)((n + 32 * s.nc - 1) / (32 * s.nc)) * ((m + 32 * s.nr - 1) / (32 * s.nr));
-        const uint64_t cost = (wgs + cus - 1) / cus * s.ns;
+    const uint32_t tiles = (m + 31) / 32;
+    for (const auto &s : kThinShapes) {
+        const uint64_t strips = (n + 32 * s.nc - 1) / (32 * s.nc);
+        /* workgroups of nr row tiles, dealt first, then one of the rest per strip */
+        const uint64_t full = strips * (tiles / s.nr), rem = full % cus;
+        uint64_t rest = tiles % s.nr ? strips : 0;
+        uint64_t cost = full / cus * thin_round(s.nc, s.nr, cus, cus);
+        if (rem) { /* the last round of full ones, and what fits beside it */
+            const uint64_t beside = rest < cus - rem ? rest : cus - rem;
+            cost += thin_round(s.nc, s.nr, rem + beside, cus);
+            rest -= beside;
+        }
+        for (; rest; rest -= rest < cus ? rest : cus) cost += thin_round(s.nc, tiles % s.nr, rest, cus);
         if (cost < best) best = cost, nr = s.nr, nc = s.nc;
     }
     return best;

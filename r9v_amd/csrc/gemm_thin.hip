@@ -23,7 +23,10 @@
  * against 0.22 us of MFMAs: its decode is 32 fma_mix (8 cycles each) and about
  * 75 other instructions a thread, and neither hides all of the other's waits.
  * A wave that decoded its own operands, without the LDS tiles, took 1.0 us;
- * four decode waves instead of eight cost 5 to 20% more at 64 columns.
+ * four decode waves instead of eight cost 5 to 20% more at 64 columns.  Eight
+ * chains a workgroup (against four) halve the decode and the weights' reads of
+ * prompt chunks: n = 4096, k = 4096 m = 777 55 -> 48 us, m = 1024 65 -> 54; they
+ * then wait on the activations, 128 KB a super-block from the L2.
  */
 #include <type_traits>
 
@@ -130,8 +133,12 @@ constexpr int thin_groups(int nc) { return kThinDec / (4 * nc); }
 /* LDS tiles: one being multiplied, the next whole, one being decoded by each group */
 constexpr int thin_tiles(int nc) { return 2 + thin_groups(nc); }
 /* 64-K steps of activations a chain holds, all but one in flight (a divisor of
- * 12: the chain's loop is unrolled over three super-blocks) */
-constexpr int thin_a_ring(int nc) { return nc == 1 ? 6 : 4; }
+ * 12: the chain's loop is unrolled over three super-blocks), and slices of B
+ * (of 16).  Eight chains make four waves a SIMD, 128 registers each: they hold
+ * less (127 used, none spilled) and cover each other's waits instead, two
+ * chains a SIMD. */
+constexpr int thin_a_ring(int nr, int nc) { return nr == 8 ? 3 : nc == 1 ? 6 : 4; }
+constexpr int thin_b_ring(int nr) { return nr == 8 ? 2 : 4; }
 
 template <int SCHEME, int NR, int NC>
 __global__ __launch_bounds__(64 * (NR + kThinDec)) void gemm_thin_kernel(ThinArgs a) {
@@ -210,16 +217,14 @@ __global__ __launch_bounds__(64 * (NR + kThinDec)) void gemm_thin_kernel(ThinArg
     }
     /* lanes past the last tile's rows read its last row again and store nothing */
     const uint32_t nk = a.k / 64, ar = (lane & 31) < rows ? (lane & 31) : rows - 1;
-    uint32_t aoff[4]; /* slice s: group 4 h + s of a step's eight */
-#pragma unroll
-    for (int s = 0; s < 4; ++s) aoff[s] = ((4 * h + s) * rows + ar) * 16;
+    const uint32_t aoff = (4 * h * rows + ar) * 16; /* slice s: group 4 h + s of a step's eight */
     const uint8_t *const abase = reinterpret_cast<const uint8_t *>(a.x16 + (uint64_t)32 * mt * a.k);
-    /* A operands, five steps ahead: x16 comes from the L2 or, on an XCD's
+    /* A operands, up to five steps ahead: x16 comes from the L2 or, on an XCD's
      * first touch, from the memory side cache, hundreds of nanoseconds away */
-    constexpr int kARing = thin_a_ring(NC);
+    constexpr int kARing = thin_a_ring(NR, NC);
     half8 af[kARing][4];
     auto load_a = [&](uint32_t step, int s, half8 &f) {
-        f = thin_ld<half8>(abase + (uint64_t)(step < nk ? step : nk - 1) * (128u * rows), aoff[s], 0);
+        f = thin_ld<half8>(abase + (uint64_t)(step < nk ? step : nk - 1) * (128u * rows) + 16u * s * rows, aoff, 0);
     };
     r9vx_f32x16 acc[NC];
 #pragma unroll
@@ -232,7 +237,8 @@ __global__ __launch_bounds__(64 * (NR + kThinDec)) void gemm_thin_kernel(ThinArg
         for (int s = 0; s < 4; ++s) load_a(i, s, af[i][s]);
         __builtin_amdgcn_sched_barrier(0); /* in the order of their use */
     }
-    half8 bf[4][NC]; /* B operands of this slice and the next three */
+    constexpr int kBRing = thin_b_ring(NR);
+    half8 bf[kBRing][NC]; /* B operands of this slice and the next ones */
     auto load_b = [&](uint32_t tile, int sl, half8 (&f)[NC]) { /* slice sl = 4 ks + s of a tile */
         const uint32_t at = tile * kTile + 64 * sl + 32 * h + ((lane & 31) ^ (2 * (sl >> 2) + h));
 #pragma unroll
@@ -249,8 +255,9 @@ __global__ __launch_bounds__(64 * (NR + kThinDec)) void gemm_thin_kernel(ThinArg
             const int ks = sl >> 2, s = sl & 3;
 #pragma unroll
             for (int ct = 0; ct < NC; ++ct)
-                acc[ct] = __builtin_amdgcn_mfma_f32_32x32x16_f16(bf[sl & 3][ct], af[(4 * j + ks) % kARing][s], acc[ct], 0, 0, 0);
-            load_b(sl < 13 ? tile : next, (sl + 3) & 15, bf[(sl + 3) & 3]); /* B(c + 1) is whole */
+                acc[ct] = __builtin_amdgcn_mfma_f32_32x32x16_f16(bf[sl % kBRing][ct], af[(4 * j + ks) % kARing][s], acc[ct], 0, 0, 0);
+            constexpr int P = kBRing - 1;
+            load_b(sl + P < 16 ? tile : next, (sl + P) & 15, bf[(sl + P) % kBRing]); /* B(c + 1) is whole */
             load_a(4 * c + ks + kARing - 1, s, af[(4 * j + ks + kARing - 1) % kARing][s]);
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -259,7 +266,7 @@ __global__ __launch_bounds__(64 * (NR + kThinDec)) void gemm_thin_kernel(ThinArg
     };
     lds_barrier(); /* B(0) and B(1) whole */
 #pragma unroll
-    for (int sl = 0; sl < 3; ++sl) load_b(0, sl, bf[sl]);
+    for (int sl = 0; sl < kBRing - 1; ++sl) load_b(0, sl, bf[sl]);
     uint32_t c0 = 0;
     for (; c0 + 3 <= nb; c0 += 3) {
 #pragma unroll
@@ -327,6 +334,7 @@ void launch_thin(const ThinArgs &a, uint32_t nr, uint32_t nc, hipStream_t s) {
     R9VX_THIN(1, 2)
     R9VX_THIN(2, 2)
     R9VX_THIN(4, 2)
+    R9VX_THIN(8, 2)
 #undef R9VX_THIN
 }
 

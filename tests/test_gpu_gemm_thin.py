@@ -58,6 +58,23 @@ def test_thin_tiles_have_the_256_row_kernels_bits(scheme):
             assert torch.equal(part.view(torch.uint8), whole[:m].view(torch.uint8)), f"m={m} out={out}"
 
 
+@pytest.mark.parametrize("scheme", SCHEMES)
+@pytest.mark.parametrize("m,k", [(577, 768), (777, 256), (1024, 512)])
+def test_eight_chain_tiles(scheme, m, k):
+    """Prompt chunks whose workgroups run eight row tiles (the last of them one,
+    part or all of it), ragged n: sampled columns against the oracle, and the
+    bits of the same rows in a launch of one and of ten row tiles."""
+    n = 4099
+    wire, w, sc = _weight(scheme, 9850, n, k)
+    x, xd = _x(9851 + m, m, k)
+    y = ffi.matmul(w, scheme, n, k, xd, w_scales=sc)
+    cols = np.r_[0:33, 2017:2051, n - 35:n]
+    rows = wire.reshape(n, -1)[cols]
+    check_close(y.cpu().numpy()[:, cols], O.matmul(scheme, np.ascontiguousarray(rows), len(cols), k, x, O.BF16), f"eight {scheme} {m}")
+    for part in (21, 300):
+        assert torch.equal(ffi.matmul(w, scheme, n, k, xd[:part], w_scales=sc), y[:part]), part
+
+
 def test_thin_tiles_under_a_captured_graph():
     """Replays of a captured launch, eager work between them, against the
     eager result, with a residual."""
