@@ -8,7 +8,7 @@
 int r9vx_launch_gemv(const r9vx_gemv_problem &p, hipStream_t stream) {
     const uint32_t cpr = p.k / 32; /* 16-byte chunks per row, a multiple of 8 */
     /* 64 lanes per row, or the power of two at or above the row's chunks when
-     * they are fewer than 33; lanes past the row's end idle (x = 0).  A row is
+     * they are fewer than 33; lanes past the row's end idle.  A row is
      * then read in one wave-wide piece per segment whatever K is: with the
      * largest power of two that divides the row's chunks instead, K = 1792 or
      * 6144 took 7 or 3 segments in series, one load latency each (Q4_K m = 6,
@@ -20,7 +20,7 @@ int r9vx_launch_gemv(const r9vx_gemv_problem &p, hipStream_t stream) {
      * choice, the rows per lane group, the activation staging and the
      * streaming forms follow m, but none of them changes a row's arithmetic: a
      * lane always owns the chunks lir, lir + 64, ... of every row and adds them
-     * in that order (two per segment or one), and the cross-lane sum over the
+     * in that order (two per segment or one; ragged rows the last first), and the cross-lane sum over the
      * 64 lanes is the same tree for every value, so a row's outputs are the
      * same bits for every m of a bucket <= 8. */
     const bool pairs = cpr % 128 == 0 || (cpr > 64 && cpr < 128);

@@ -46,7 +46,7 @@ struct GemvArgs {
     uint32_t k;
     uint32_t lpr_log2; /* lanes per row = 1 << lpr_log2 */
     uint32_t nseg;     /* K segments of LPR*SPL chunks */
-    uint32_t cpr;      /* chunks per row: a lane whose chunk is past them repeats the last with x = 0 */
+    uint32_t cpr;      /* chunks per row: a lane whose chunk is past them repeats the last and drops it */
     uint32_t ragged;   /* cpr is not a whole number of segments */
     uint32_t y_bf16;
     uint32_t epilogue;
@@ -78,21 +78,30 @@ constexpr int waves_for(int m) { return m <= 2 ? 2 : 1; }
 
 using namespace r9vx;
 
-/* x = 0 for the chunk of a lane past the row's end: its products add nothing. */
-template <bool XF32>
-__device__ __forceinline__ void mask_x(XRaw<XF32> &r, bool live) {
+/* What a kernel's rows and outputs are: */
+enum RowForm {
+    kPlain,  /* rows that fill their K segments; the 64-lane forms: f32 y, no epilogue */
+    kEpi,    /* 64-lane forms: the same rows, the epilogue and y's type read from the arguments */
+    kRagged, /* rows whose chunks do not fill the last K segment (epilogue as kEpi) */
+};
+
+/* Ragged rows: lanes past the row's end repeat its last chunk, so that every
+ * load stays in the row, and what they summed is dropped.  (With x = 0 there
+ * instead, an infinite block scale of that chunk would make the row NaN.)  The
+ * row's last segment goes first, the last of a lane's chunks first in it: the
+ * lanes' sums are then only those of the repeated chunk, and one select per sum
+ * drops them, without a copy of the sums so far.  Selects on the activations
+ * took more (Q4_K m = 8, n = 16384, K = 4352 53.0 -> 42.4 us; Q8_0 61.6 -> 53.2;
+ * one segment, K = 1280, the same). */
+template <int M>
+__device__ __forceinline__ void drop_idle(bool live, float (&acc)[M]) {
 #pragma unroll
-    for (int i = 0; i < (XF32 ? 8 : 4); ++i)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) r.v[i][e] = live ? r.v[i][e] : 0;
+    for (int t = 0; t < M; ++t) acc[t] = live ? acc[t] : 0.f;
 }
 
-/* RAG: the row's chunks do not fill its segments (or, LPRL = 6, the launch has
- * an epilogue or bf16 outputs): lanes past the row's end repeat its last chunk
- * with x = 0, and the epilogue is read from the arguments.  A kernel of its
- * own: the selects cost full rows 3% (n = 5120, K = 2048, M = 5: 4.71 -> 4.86
- * us) to 28% (gated, K = 4096, M = 6).
- * LPRL = 6: 64 lanes per row and a single K segment (K = 2048*SPL; RAG: up to
+/* FORM (RowForm): ragged rows have kernels of their own, so that full rows carry
+ * neither the selects nor the bounds of the loads.
+ * LPRL = 6: 64 lanes per row and a single K segment (K = 2048*SPL; kRagged: up to
  * that), fixed at compile time (measured 0.4-0.6 us faster per launch at n = 5120, K = 2048
  * than the general form), and RR rows per lane group
  * chosen by the launcher to balance the waves over the SIMDs (NS = 0: the
@@ -105,9 +114,10 @@ __device__ __forceinline__ void mask_x(XRaw<XF32> &r, bool live) {
  * ((s M + t) NP + j) 64 + l, so each wave's 16-byte reads are contiguous
  * across its lanes) and every wave reads its slices from there, instead of
  * each wave loading all of x from L2. */
-template <int SCHEME, int M, bool XF32, int SPL, int LPRL, int RR, int NS, bool XS, bool RAG>
+template <int SCHEME, int M, bool XF32, int SPL, int LPRL, int RR, int NS, bool XS, int FORM>
 __global__ __launch_bounds__(XS ? 256 : waves_for(M) * 64) void gemv_kernel(GemvArgs a) {
     static_assert(!XS || (LPRL == 6 && NS == 1), "x staging needs the single-segment 64-lane form");
+    constexpr bool RAG = FORM == kRagged;
     constexpr int kRows = RR ? RR : rows_for(M), kWaves = XS ? 4 : waves_for(M);
     constexpr int kNP = XF32 ? 8 : 4; /* 16-byte pieces of a lane's chunk of one x row */
     constexpr int kPieces = XS ? SPL * M * kNP * 64 : 1;
@@ -130,7 +140,8 @@ __global__ __launch_bounds__(XS ? 256 : waves_for(M) * 64) void gemv_kernel(Gemv
         for (int t = 0; t < M; ++t) acc[r][t] = 0.f;
 
     const uint32_t nseg = (LPRL && NS == 1) ? 1u : a.nseg;
-    for (uint32_t seg = 0; seg < nseg; ++seg) {
+    for (uint32_t i = 0; i < nseg; ++i) {
+        const uint32_t seg = RAG ? nseg - 1 - i : i;
         uint32_t cis[SPL];
         bool live[SPL];
 #pragma unroll
@@ -160,7 +171,6 @@ __global__ __launch_bounds__(XS ? 256 : waves_for(M) * 64) void gemv_kernel(Gemv
                     const uint8_t *xb = reinterpret_cast<const uint8_t *>(a.x) +
                                         ((uint64_t)t * a.x_row_stride + e) * (XF32 ? 4 : 2);
                     xst[q] = *reinterpret_cast<const r9vx_u32x4 *>(xb);
-                    if (RAG && ci >= a.cpr) xst[q] = r9vx_u32x4{0u, 0u, 0u, 0u};
                 }
             }
         } else {
@@ -201,12 +211,12 @@ __global__ __launch_bounds__(XS ? 256 : waves_for(M) * 64) void gemv_kernel(Gemv
         /* 2. the codebook table is built (and the activation copy stored)
          * while the weight loads are in flight */
         if constexpr (SCHEME == R9VX_SCHEME_IQ4_XS) {
-            if ((LPRL != 0 && NS == 1) || seg == 0) {
+            if ((LPRL != 0 && NS == 1) || i == 0) {
                 build_iq4_lut(lut, threadIdx.x, blockDim.x);
                 if constexpr (!XS) __syncthreads();
             }
         } else if constexpr (SCHEME == R9VX_SCHEME_IQ3_S) {
-            if ((LPRL != 0 && NS == 1) || seg == 0) {
+            if ((LPRL != 0 && NS == 1) || i == 0) {
                 build_iq3s_lut(lut, threadIdx.x, blockDim.x);
                 if constexpr (!XS) __syncthreads();
             }
@@ -231,12 +241,6 @@ __global__ __launch_bounds__(XS ? 256 : waves_for(M) * 64) void gemv_kernel(Gemv
                             xr[s][t].v[j] = v;
                     }
         }
-        if constexpr (RAG && !XS) { /* (the staged copy holds zeros there) */
-#pragma unroll
-            for (int s = 0; s < SPL; ++s)
-#pragma unroll
-                for (int t = 0; t < M; ++t) mask_x<XF32>(xr[s][t], live[s]);
-        }
         XChunk<SCHEME, XF32> xc[SPL][M];
 #pragma unroll
         for (int s = 0; s < SPL; ++s)
@@ -245,14 +249,20 @@ __global__ __launch_bounds__(XS ? 256 : waves_for(M) * 64) void gemv_kernel(Gemv
 #pragma unroll
         for (int r = 0; r < kRows; ++r)
 #pragma unroll
-            for (int s = 0; s < SPL; ++s) {
+            for (int j = 0; j < SPL; ++j) {
+                const int s = RAG ? SPL - 1 - j : j;
                 if constexpr (SCHEME == R9VX_SCHEME_IQ3_S)
                     chunk_dot_iq3s<M>(qs[r][s], hd[r][s], cis[s] & 7, xc[s], acc[r], lut);
                 else if constexpr (split_scheme(SCHEME))
                     chunk_dot_split<SCHEME, M>(qs[r][s], hd[r][s], cis[s] & 7, xc[s], acc[r]);
                 else
                     chunk_dot<SCHEME, XF32, M>(qs[r][s], hd[r][s], cis[s] & 7, xc[s], acc[r], lut);
+                if constexpr (RAG && SPL == 2) drop_idle<M>(live[s], acc[r]); /* then nseg = 1 */
             }
+        if constexpr (RAG && SPL == 1)
+            if (i == 0)
+#pragma unroll
+                for (int r = 0; r < kRows; ++r) drop_idle<M>(live[0], acc[r]);
     }
 
     /* cross-lane sums of all kRows*M partials at once; the lanes that end
@@ -268,7 +278,7 @@ __global__ __launch_bounds__(XS ? 256 : waves_for(M) * 64) void gemv_kernel(Gemv
         const uint32_t row = row0 + r * rpi;
         if (row >= a.n) return;
         float y = val[0];
-        if constexpr (LPRL != 0 && !RAG) {
+        if constexpr (LPRL != 0 && FORM == kPlain) {
             reinterpret_cast<float *>(a.y)[(uint64_t)t * a.n + row] = y;
             return;
         }
@@ -296,14 +306,15 @@ __global__ __launch_bounds__(XS ? 256 : waves_for(M) * 64) void gemv_kernel(Gemv
  * sums wait in LDS until the wave's last load is issued: a store between
  * two loads would make the next wait a wait for the store as well.  Per row
  * the arithmetic is gemv_kernel's (the lane's chunks lir, lir + 64 in that
- * order, the same cross-lane tree), so the outputs are the same bits. */
+ * order, or for ragged rows the other; the same cross-lane tree), so the outputs
+ * are the same bits. */
 constexpr uint32_t kStreamMaxSteps = 16;
 /* rows per group and waves per SIMD: measured (Q4_K 32768 x 4096, IQ4_XS
  * 32768 x 2048, Q4_K 14336 x 4096, graph-replayed) against (2, 3), (4, 2),
  * (1, 4), (2, 4) and (4, 3), which were 2-50% slower */
 constexpr uint32_t kStreamRows = 2, kStreamWavesPerSimd = 2;
 
-template <int SCHEME, bool XF32, int SPL, int RR>
+template <int SCHEME, bool XF32, int SPL, int RR, bool RAG>
 __global__ __launch_bounds__(256) void gemv_stream_kernel(GemvArgs a, uint32_t steps) {
     using Pay = typename std::conditional<pay2_scheme(SCHEME), Payload2, r9vx_u32x4>::type;
     __shared__ __attribute__((aligned(16))) uint32_t lut[lut_words(SCHEME)];
@@ -312,8 +323,13 @@ __global__ __launch_bounds__(256) void gemv_stream_kernel(GemvArgs a, uint32_t s
     const uint32_t gw = blockIdx.x * 4 + wl, nw = gridDim.x * 4;
     const uint32_t ngroups = (a.n + RR - 1) / RR;
     uint32_t cis[SPL];
+    bool live[SPL];
 #pragma unroll
-    for (int s = 0; s < SPL; ++s) cis[s] = (uint32_t)s * 64u + lane < a.cpr ? (uint32_t)s * 64u + lane : a.cpr - 1;
+    for (int s = 0; s < SPL; ++s) {
+        const uint32_t ci = (uint32_t)s * 64u + lane;
+        live[s] = !RAG || ci < a.cpr;
+        cis[s] = live[s] ? ci : a.cpr - 1;
+    }
     XRaw<XF32> xr[SPL];
 #pragma unroll
     for (int s = 0; s < SPL; ++s) {
@@ -321,8 +337,6 @@ __global__ __launch_bounds__(256) void gemv_stream_kernel(GemvArgs a, uint32_t s
         chunk_k<SCHEME>(cis[s], klo, khi);
         load_x_raw<XF32>(a.x, klo, khi, xr[s]);
     }
-#pragma unroll
-    for (int s = 0; s < SPL; ++s) mask_x<XF32>(xr[s], (uint32_t)s * 64u + lane < a.cpr);
     __builtin_amdgcn_sched_barrier(0);
     Pay qa[RR][SPL], qb[RR][SPL];
     Hdr ha[RR][SPL], hb[RR][SPL];
@@ -352,7 +366,11 @@ __global__ __launch_bounds__(256) void gemv_stream_kernel(GemvArgs a, uint32_t s
         for (int r = 0; r < RR; ++r) {
             acc[r][0] = 0.f;
 #pragma unroll
-            for (int s = 0; s < SPL; ++s) chunk_dot<SCHEME, XF32, 1>(q[r][s], h[r][s], cis[s] & 7, xc[s], acc[r], lut);
+            for (int j = 0; j < SPL; ++j) {
+                const int s = RAG ? SPL - 1 - j : j;
+                chunk_dot<SCHEME, XF32, 1>(q[r][s], h[r][s], cis[s] & 7, xc[s], acc[r], lut);
+                if constexpr (RAG) drop_idle<1>(live[s], acc[r]);
+            }
         }
         float v[1][RR];
 #pragma unroll
@@ -382,7 +400,10 @@ int launch_stream(const GemvArgs &a, uint32_t simds, hipStream_t s) {
     uint32_t waves = kStreamWavesPerSimd * simds;
     if ((ngroups + waves - 1) / waves > kStreamMaxSteps) waves = (ngroups + kStreamMaxSteps - 1) / kStreamMaxSteps;
     const uint32_t wgs = (waves + 3) / 4, steps = (ngroups + wgs * 4 - 1) / (wgs * 4);
-    hipLaunchKernelGGL((gemv_stream_kernel<SCHEME, XF32, SPL, kStreamRows>), dim3(wgs), dim3(256), 0, s, a, steps);
+    if (a.ragged)
+        hipLaunchKernelGGL((gemv_stream_kernel<SCHEME, XF32, SPL, kStreamRows, true>), dim3(wgs), dim3(256), 0, s, a, steps);
+    else
+        hipLaunchKernelGGL((gemv_stream_kernel<SCHEME, XF32, SPL, kStreamRows, false>), dim3(wgs), dim3(256), 0, s, a, steps);
     return (int)hipGetLastError();
 }
 
@@ -416,7 +437,8 @@ __global__ __launch_bounds__(waves_for(M) * 64) void gemv_gated_kernel(GemvArgs 
 #pragma unroll
             for (int t = 0; t < M; ++t) acc[h][r][t] = 0.f;
 
-    for (uint32_t seg = 0; seg < a.nseg; ++seg) {
+    for (uint32_t i = 0; i < a.nseg; ++i) {
+        const uint32_t seg = RAG ? a.nseg - 1 - i : i;
         uint32_t cis[SPL];
         bool live[SPL];
 #pragma unroll
@@ -457,12 +479,12 @@ __global__ __launch_bounds__(waves_for(M) * 64) void gemv_gated_kernel(GemvArgs 
                 }
             }
         if constexpr (SCHEME == R9VX_SCHEME_IQ4_XS) {
-            if (seg == 0) {
+            if (i == 0) {
                 build_iq4_lut(lut, threadIdx.x, blockDim.x);
                 __syncthreads();
             }
         } else if constexpr (SCHEME == R9VX_SCHEME_IQ3_S) {
-            if (seg == 0) {
+            if (i == 0) {
                 build_iq3s_lut(lut, threadIdx.x, blockDim.x);
                 __syncthreads();
             }
@@ -471,22 +493,28 @@ __global__ __launch_bounds__(waves_for(M) * 64) void gemv_gated_kernel(GemvArgs 
 #pragma unroll
         for (int s = 0; s < SPL; ++s)
 #pragma unroll
-            for (int t = 0; t < M; ++t) {
-                if constexpr (RAG) mask_x<false>(xr[s][t], live[s]);
-                arrange_x<SCHEME, false>(xr[s][t], xc[s][t]);
-            }
+            for (int t = 0; t < M; ++t) arrange_x<SCHEME, false>(xr[s][t], xc[s][t]);
 #pragma unroll
         for (int h = 0; h < 2; ++h)
 #pragma unroll
             for (int r = 0; r < kRows; ++r)
 #pragma unroll
-                for (int s = 0; s < SPL; ++s) {
+                for (int j = 0; j < SPL; ++j) {
+                    const int s = RAG ? SPL - 1 - j : j;
                     if constexpr (SCHEME == R9VX_SCHEME_IQ3_S)
                         chunk_dot_iq3s<M>(qs[h][r][s], hd[h][r][s], cis[s] & 7, xc[s], acc[h][r], lut);
                     else if constexpr (split_scheme(SCHEME))
                         chunk_dot_split<SCHEME, M>(qs[h][r][s], hd[h][r][s], cis[s] & 7, xc[s], acc[h][r]);
                     else
                         chunk_dot<SCHEME, false, M>(qs[h][r][s], hd[h][r][s], cis[s] & 7, xc[s], acc[h][r], lut);
+                    if constexpr (RAG && SPL == 2) drop_idle<M>(live[s], acc[h][r]); /* then nseg = 1 */
+                }
+        if constexpr (RAG && SPL == 1)
+            if (i == 0)
+#pragma unroll
+                for (int r = 0; r < kRows; ++r) {
+                    drop_idle<M>(live[0], acc[0][r]);
+                    drop_idle<M>(live[0], acc[1][r]);
                 }
     }
 
@@ -525,7 +553,7 @@ __global__ __launch_bounds__(waves_for(M) * 64) void gemv_gated_kernel(GemvArgs 
  * n = 2816, K = 2048, m = 1: 4.44 against 4.76 us). */
 constexpr uint32_t kGatedMaxSteps = 16;
 
-template <int SCHEME, int M, int SPL>
+template <int SCHEME, int M, int SPL, bool RAG>
 __global__ __launch_bounds__(256) void gemv_gated_stream_kernel(GemvArgs a, uint32_t steps) {
     using Pay = typename std::conditional<pay2_scheme(SCHEME), Payload2, r9vx_u32x4>::type;
     __shared__ __attribute__((aligned(16))) uint32_t lut[lut_words(SCHEME)];
@@ -533,10 +561,13 @@ __global__ __launch_bounds__(256) void gemv_gated_stream_kernel(GemvArgs a, uint
     const uint32_t lane = threadIdx.x & 63, wl = threadIdx.x >> 6;
     const uint32_t gw = blockIdx.x * 4 + wl, nw = gridDim.x * 4;
     uint32_t cis[SPL];
+    bool live[SPL];
     XRaw<false> xr[SPL][M];
 #pragma unroll
     for (int s = 0; s < SPL; ++s) {
-        cis[s] = (uint32_t)s * 64u + lane < a.cpr ? (uint32_t)s * 64u + lane : a.cpr - 1;
+        const uint32_t ci = (uint32_t)s * 64u + lane;
+        live[s] = !RAG || ci < a.cpr;
+        cis[s] = live[s] ? ci : a.cpr - 1;
         uint32_t klo, khi;
         chunk_k<SCHEME>(cis[s], klo, khi);
 #pragma unroll
@@ -575,10 +606,7 @@ __global__ __launch_bounds__(256) void gemv_gated_stream_kernel(GemvArgs a, uint
 #pragma unroll
     for (int s = 0; s < SPL; ++s)
 #pragma unroll
-        for (int t = 0; t < M; ++t) {
-            mask_x<false>(xr[s][t], (uint32_t)s * 64u + lane < a.cpr);
-            arrange_x<SCHEME, false>(xr[s][t], xc[s][t]);
-        }
+        for (int t = 0; t < M; ++t) arrange_x<SCHEME, false>(xr[s][t], xc[s][t]);
     float *const obw = ob[wl];
     auto compute = [&](uint32_t step, const Pay (&q)[2][SPL], const Hdr (&h)[2][SPL]) {
         float v[2][M];
@@ -587,13 +615,15 @@ __global__ __launch_bounds__(256) void gemv_gated_stream_kernel(GemvArgs a, uint
 #pragma unroll
             for (int t = 0; t < M; ++t) v[g][t] = 0.f;
 #pragma unroll
-            for (int s = 0; s < SPL; ++s) {
+            for (int j = 0; j < SPL; ++j) {
+                const int s = RAG ? SPL - 1 - j : j;
                 if constexpr (SCHEME == R9VX_SCHEME_IQ3_S)
                     chunk_dot_iq3s<M>(q[g][s], h[g][s], cis[s] & 7, xc[s], v[g], lut);
                 else if constexpr (split_scheme(SCHEME))
                     chunk_dot_split<SCHEME, M>(q[g][s], h[g][s], cis[s] & 7, xc[s], v[g]);
                 else
                     chunk_dot<SCHEME, false, M>(q[g][s], h[g][s], cis[s] & 7, xc[s], v[g], lut);
+                if constexpr (RAG) drop_idle<M>(live[s], v[g]);
             }
         }
         lane_reduce<M, 64, 2>(v, lane, [&](int t, const float (&val)[2]) {
@@ -633,7 +663,10 @@ int launch_gated_stream(const GemvArgs &a, uint32_t m, uint32_t simds, hipStream
         if (waves > a.n) waves = a.n;
         if ((a.n + waves - 1) / waves > kGatedMaxSteps) waves = (a.n + kGatedMaxSteps - 1) / kGatedMaxSteps;
         const uint32_t wgs = (waves + 3) / 4, steps = (a.n + wgs * 4 - 1) / (wgs * 4);
-        hipLaunchKernelGGL((gemv_gated_stream_kernel<SCHEME, MM, SPL>), dim3(wgs), dim3(256), 0, s, a, steps);
+        if (a.ragged)
+            hipLaunchKernelGGL((gemv_gated_stream_kernel<SCHEME, MM, SPL, true>), dim3(wgs), dim3(256), 0, s, a, steps);
+        else
+            hipLaunchKernelGGL((gemv_gated_stream_kernel<SCHEME, MM, SPL, false>), dim3(wgs), dim3(256), 0, s, a, steps);
         return (int)hipGetLastError();
     }
 }
@@ -702,11 +735,16 @@ int launch_rows(const GemvArgs &a, uint32_t rows_per_slot_group, hipStream_t s) 
     const uint32_t waves = (a.n + rows_per_wave - 1) / rows_per_wave;
     const uint32_t wpg = XS ? 4 : waves_for(MM);
     const dim3 grid((waves + wpg - 1) / wpg);
-    const bool plain = a.epilogue == R9VX_EPILOGUE_NONE && !a.y_bf16;
-    if (a.ragged || (LPRL != 0 && !plain))
-        hipLaunchKernelGGL((gemv_kernel<SCHEME, MM, XF32, SPL, LPRL, RR, NS, XS, true>), grid, dim3(wpg * 64), 0, s, a);
+    if constexpr (LPRL != 0 && NS == 1) {
+        if (!a.ragged && (a.epilogue != R9VX_EPILOGUE_NONE || a.y_bf16)) {
+            hipLaunchKernelGGL((gemv_kernel<SCHEME, MM, XF32, SPL, LPRL, RR, NS, XS, kEpi>), grid, dim3(wpg * 64), 0, s, a);
+            return (int)hipGetLastError();
+        }
+    }
+    if (a.ragged)
+        hipLaunchKernelGGL((gemv_kernel<SCHEME, MM, XF32, SPL, LPRL, RR, NS, XS, kRagged>), grid, dim3(wpg * 64), 0, s, a);
     else
-        hipLaunchKernelGGL((gemv_kernel<SCHEME, MM, XF32, SPL, LPRL, RR, NS, XS, false>), grid, dim3(wpg * 64), 0, s, a);
+        hipLaunchKernelGGL((gemv_kernel<SCHEME, MM, XF32, SPL, LPRL, RR, NS, XS, kPlain>), grid, dim3(wpg * 64), 0, s, a);
     return (int)hipGetLastError();
 }
 

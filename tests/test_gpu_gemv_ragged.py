@@ -74,3 +74,40 @@ def test_gated_streaming_form_has_the_one_shot_forms_bits(scheme, n, k):
         y16 = ffi.matmul(w, scheme, n, k, xd[:m], w_scales=sc, swiglu=True, out_dtype=ffi.BF16)
         assert torch.equal(y16, y.to(torch.bfloat16))
         assert torch.equal(ffi.matmul(w, scheme, n, k, xd[m - 1:m], w_scales=sc, swiglu=True)[0], y[m - 1])
+
+
+def _last_block_infinite(scheme, wire, n, k):
+    """The last block of every row of `wire`, made of positive weights under an infinite scale."""
+    w = wire.reshape(n, k // ffi.BLOCK_LEN[scheme], -1)
+    last = w[:, -1]
+    if scheme == O.Q8_0:  # quants 1
+        last[:, 2:] = 1
+    elif scheme == O.IQ4_XS:  # sub-block scales 63 - 32, the codebook's largest value
+        last[:, 2:] = 0xFF
+    elif scheme == O.Q6_K:  # quants 63 - 32, sub-block scales 1
+        last[:, :192], last[:, 192:208] = 0xFF, 1
+    else:  # IQ3_S: no signs (the codebook's values are positive)
+        last[:, 74:106] = 0
+    at = 208 if scheme == O.Q6_K else 0
+    last[:, at:at + 2] = np.frombuffer(np.float16(np.inf).tobytes(), np.uint8)
+    return w.reshape(wire.shape)
+
+
+# n, K, m, gated: one and several segments, one and two chunks a lane, the streaming forms, full rows
+INFINITE = [(5, 768, 1, False), (70, 2304, 3, False), (70, 2304, 8, False), (33, 6400, 5, False), (33, 2816, 2, True),
+            (20, 4352, 6, True), (8200, 1280, 3, True), (12300, 1280, 1, False), (5, 2048, 1, False)]
+
+
+@pytest.mark.parametrize("scheme,n,k,m,swiglu,x_f32",
+                         [(s, *c, False) for s in (O.IQ4_XS, O.Q6_K, O.Q8_0, O.IQ3_S) for c in INFINITE]
+                         + [(O.IQ4_XS, 40, 3840, 2, False, True), (O.IQ4_XS, 9, 768, 1, False, True)])
+def test_infinite_last_block_is_not_nan(scheme, n, k, m, swiglu, x_f32):
+    """Lanes past a ragged row's end read its last block again: its infinite
+    scale must stay the row's infinity, as in rows that fill their segments."""
+    rows = 2 * n if swiglu else n
+    wire = _last_block_infinite(scheme, synth.quant_weights(scheme, 9970 + k, rows, k).copy(), rows, k)
+    w = torch.from_numpy(wire.reshape(-1)).cuda()
+    w, sc = (w, None) if scheme == O.IQ4_XS else ffi.repack(w, scheme, rows, k)
+    x = torch.ones((m, k), dtype=torch.float32 if x_f32 else torch.bfloat16, device="cuda")
+    y = ffi.matmul(w, scheme, n, k, x, w_scales=sc, swiglu=swiglu)
+    assert bool((y == float("inf")).all())
