@@ -371,8 +371,18 @@ constexpr uint32_t kRouteSmallT = 8;
 constexpr uint32_t kRouteMidT = 128;
 /* and up to this many logits, past which the workgroups' reads cost more than
  * the launches: E = 512 T = 96 11.4 -> 8.7 us, T = 128 11.5 / 11.0; E = 1024
- * T = 48 16.5 -> 10.1, T = 96 16.7 / 17.2; E = 64 T = 128 7.2 -> 5.2 */
+ * T = 48 16.5 -> 10.1, T = 96 16.7 / 17.2; E = 64 T = 128 7.2 -> 5.2.  From E =
+ * 257 the rows take registers for 512 scores each, and 96 rows are the line (E =
+ * 300, K = 2: T = 96 9.5 -> 8.9, T = 128 9.5 / 11.0). */
 constexpr uint32_t kRouteMidLogits = 48u << 10;
+constexpr uint32_t route_mid_softmax_t(int per) { return per >= 8 ? 96 : kRouteMidT; }
+/* Sigmoid scores: the check needs every value's exp, not only the row's maximum,
+ * and every workgroup repeats it, so the launches are the cheaper already at
+ * fewer rows (PER = ceil(E / 64) to a power of two; K = 8, three launches / one):
+ * E = 64 T = 48 7.3 / 6.7 us, T = 64 7.3 / 7.6; E = 256 T = 32 8.3 / 7.2, T = 48
+ * 8.3 / 8.5; E = 512 T = 24 9.5 / 8.2, T = 32 9.6 / 9.5, T = 96 9.8 / 17.5;
+ * E = 1024 T = 16 13.5 / 11.2, T = 32 13.8 / 15.9. */
+constexpr uint32_t route_mid_sigmoid_t(int per) { return per <= 2 ? 48 : per == 4 ? 32 : per == 8 ? 24 : 16; }
 constexpr uint32_t kRouteCheckRows = 4; /* rows a checking wave loads at once */
 
 /* Rows first, first + STRIDE, ...: R of them. */
@@ -674,7 +684,8 @@ static int launch_route_per(const RouteArgs &a, hipStream_t stream) {
         hipLaunchKernelGGL((route_small_kernel<PER, 2>), dim3(a.t), dim3(256), 0, stream, a);
         return (int)hipGetLastError();
     }
-    if (a.t <= kRouteMidT && a.t * a.e <= kRouteMidLogits) {
+    const uint32_t mid = a.scoring == R9VX_SCORING_SIGMOID ? route_mid_sigmoid_t(PER) : route_mid_softmax_t(PER);
+    if (a.t <= mid && a.t * a.e <= kRouteMidLogits) {
         hipLaunchKernelGGL((route_small_kernel<PER, 6>), dim3(a.t), dim3(512), 0, stream, a);
         return (int)hipGetLastError();
     }

@@ -34,3 +34,17 @@ def test_route_mid_refuses_before_writing(t):
         ffi.moe_route(torch.from_numpy(z).cuda(), 4, ids=ids, weights=w, status=status)
         assert ffi.status_read(status) == ffi.STATUS_NONFINITE, f"bad row {bad}"
         assert bool((ids == -7).all()) and bool((w == -7.0).all())
+
+
+@pytest.mark.parametrize("scoring,e,line", [(ffi.SCORING_SIGMOID, 128, 48), (ffi.SCORING_SIGMOID, 256, 32),
+                                            (ffi.SCORING_SIGMOID, 512, 24), (ffi.SCORING_SIGMOID, 1024, 16),
+                                            (ffi.SCORING_SOFTMAX, 300, 96)])
+def test_route_mid_lines_with_a_bias(scoring, e, line):
+    """Both sides of the row count up to which one launch routes."""
+    bias = synth.normal_f32(9350 + e, (e,))
+    for t in (line, line + 1):
+        z = synth.normal_f32(9360 + t + e, (t, e))
+        ids, w = ffi.moe_route(torch.from_numpy(z).cuda(), 6, bias=torch.from_numpy(bias).cuda(), scoring=scoring)
+        ids_o, w_o = O.moe_route(z, 6, bias=bias, scoring=scoring)
+        assert np.array_equal(ids.cpu().numpy().view(np.uint32), ids_o)
+        assert np.array_equal(w.cpu().numpy().view(np.uint32), w_o.view(np.uint32))

@@ -1,0 +1,40 @@
+"""Which kernels the library launches for a call, and with what grids, recorded
+on the CPU (tests/launch_record.py): the dispatch rules' lines, and HIP's limits
+on a launch."""
+from __future__ import annotations
+
+import shutil
+
+import pytest
+
+import launch_record
+from r9v_amd import ffi
+
+pytestmark = pytest.mark.skipif(not launch_record.LIB.exists() or shutil.which("gcc") is None,
+                                reason="needs the built libr9vx.so and gcc")
+
+
+@pytest.fixture(scope="module")
+def runtime(tmp_path_factory):
+    return launch_record.build(tmp_path_factory.mktemp("hip"))
+
+
+def kernels(runtime, calls):
+    out = launch_record.record(runtime, calls)
+    assert all(rc == 0 for rc, _, _ in out), out
+    return [[k for k, _, _ in launches] for _, _, launches in out]
+
+
+# experts, scores, the most rows that one launch routes: past them checking every
+# row in every workgroup costs more than the launches that it saves
+ROUTE_LINES = [(64, ffi.SCORING_SOFTMAX, 128), (256, ffi.SCORING_SOFTMAX, 128), (300, ffi.SCORING_SOFTMAX, 96),
+               (512, ffi.SCORING_SOFTMAX, 96), (768, ffi.SCORING_SOFTMAX, 64), (1024, ffi.SCORING_SOFTMAX, 48),
+               (64, ffi.SCORING_SIGMOID, 48), (128, ffi.SCORING_SIGMOID, 48), (256, ffi.SCORING_SIGMOID, 32),
+               (512, ffi.SCORING_SIGMOID, 24), (768, ffi.SCORING_SIGMOID, 16), (1024, ffi.SCORING_SIGMOID, 16)]
+
+
+@pytest.mark.parametrize("e,scoring,line", ROUTE_LINES)
+def test_router_launches(runtime, e, scoring, line):
+    last, past = kernels(runtime, [("route", dict(t=t, e=e, k=8, scoring=scoring)) for t in (line, line + 1)])
+    assert len(last) == 1 and last[0].startswith("route_small_kernel")
+    assert [k.split("<")[0] for k in past] == ["clear_status_kernel", "route_check_kernel", "route_kernel"]
