@@ -323,6 +323,12 @@ __global__ __launch_bounds__(64 * (NR + kThinDec)) void gemm_thin_kernel(ThinArg
         }
 }
 
+/* Rows of one launch: a multiple of every shape's row tiles whose grids stay
+ * within HIP's limits (2^32 threads in x, one workgroup of 256 per row in the
+ * conversion; 65535 workgroups in y, 32 rows each and more).  Which rows share a
+ * launch changes no output bit. */
+constexpr uint32_t kThinMaxRows = 1u << 20;
+
 template <int SCHEME>
 void launch_thin(const ThinArgs &a, uint32_t nr, uint32_t nc, hipStream_t s) {
     const dim3 grid((a.n + 32 * nc - 1) / (32 * nc), (a.m + 32 * nr - 1) / (32 * nr)), block(64 * (nr + kThinDec));
@@ -338,6 +344,16 @@ void launch_thin(const ThinArgs &a, uint32_t nr, uint32_t nc, hipStream_t s) {
 #undef R9VX_THIN
 }
 
+void launch_x16(uint32_t order, const uint16_t *x, uint32_t m, uint32_t k, _Float16 *x16, float *scale, hipStream_t s) {
+    const dim3 grid(m), block(256);
+    switch (order) {
+    case R9VX_SCHEME_Q4_K: hipLaunchKernelGGL(x_to_f16_thin_kernel<R9VX_SCHEME_Q4_K>, grid, block, 0, s, x, m, k, x16, scale); break;
+    case R9VX_SCHEME_IQ4_XS: hipLaunchKernelGGL(x_to_f16_thin_kernel<R9VX_SCHEME_IQ4_XS>, grid, block, 0, s, x, m, k, x16, scale); break;
+    case R9VX_SCHEME_Q6_K: hipLaunchKernelGGL(x_to_f16_thin_kernel<R9VX_SCHEME_Q6_K>, grid, block, 0, s, x, m, k, x16, scale); break;
+    default: hipLaunchKernelGGL(x_to_f16_thin_kernel<0>, grid, block, 0, s, x, m, k, x16, scale); break;
+    }
+}
+
 }  // namespace
 
 int r9vx_launch_gemm_thin(const r9vx_gemm_problem &p, uint32_t nr, uint32_t nc, hipStream_t stream) {
@@ -345,32 +361,31 @@ int r9vx_launch_gemm_thin(const r9vx_gemm_problem &p, uint32_t nr, uint32_t nc, 
     _Float16 *x16 = reinterpret_cast<_Float16 *>(p.workspace);
     float *scale = reinterpret_cast<float *>(reinterpret_cast<uint8_t *>(p.workspace) +
                                              r9vx_gemm_x16_bytes(p.m, p.k));
-    a.x16 = x16;
-    a.scale = scale;
     a.w = p.w;
     a.ws = p.w_scales;
     a.bias = p.bias;
-    a.residual = p.residual;
-    a.y = p.y;
     a.w_row_stride = r9vx_row_bytes(p.scheme, p.k);
     a.ws_row = r9vx_row_scales(p.scheme, p.k);
-    a.m = p.m;
     a.n = p.n;
     a.k = p.k;
     a.y_bf16 = p.y_dtype == R9VX_DTYPE_BF16;
     a.epilogue = p.epilogue;
-    switch (r9vx_group_order(p.scheme)) {
-    case R9VX_SCHEME_Q4_K: hipLaunchKernelGGL(x_to_f16_thin_kernel<R9VX_SCHEME_Q4_K>, dim3(p.m), dim3(256), 0, stream, p.x, p.m, p.k, x16, scale); break;
-    case R9VX_SCHEME_IQ4_XS: hipLaunchKernelGGL(x_to_f16_thin_kernel<R9VX_SCHEME_IQ4_XS>, dim3(p.m), dim3(256), 0, stream, p.x, p.m, p.k, x16, scale); break;
-    case R9VX_SCHEME_Q6_K: hipLaunchKernelGGL(x_to_f16_thin_kernel<R9VX_SCHEME_Q6_K>, dim3(p.m), dim3(256), 0, stream, p.x, p.m, p.k, x16, scale); break;
-    default: hipLaunchKernelGGL(x_to_f16_thin_kernel<0>, dim3(p.m), dim3(256), 0, stream, p.x, p.m, p.k, x16, scale); break;
+    for (uint32_t r0 = 0; r0 < p.m; r0 += kThinMaxRows) {
+        a.m = p.m - r0 < kThinMaxRows ? p.m - r0 : kThinMaxRows;
+        a.x16 = x16 + (size_t)r0 * p.k;
+        a.scale = scale + r0;
+        a.residual = p.residual ? p.residual + (size_t)r0 * p.n : nullptr;
+        a.y = reinterpret_cast<uint8_t *>(p.y) + (size_t)r0 * p.n * (a.y_bf16 ? 2 : 4);
+        launch_x16(r9vx_group_order(p.scheme), p.x + (size_t)r0 * p.k, a.m, p.k, x16 + (size_t)r0 * p.k, scale + r0, stream);
+        switch (p.scheme) {
+        case R9VX_SCHEME_Q4_K: launch_thin<R9VX_SCHEME_Q4_K>(a, nr, nc, stream); break;
+        case R9VX_SCHEME_IQ4_XS: launch_thin<R9VX_SCHEME_IQ4_XS>(a, nr, nc, stream); break;
+        case R9VX_SCHEME_Q6_K: launch_thin<R9VX_SCHEME_Q6_K>(a, nr, nc, stream); break;
+        case R9VX_SCHEME_Q8_0: launch_thin<R9VX_SCHEME_Q8_0>(a, nr, nc, stream); break;
+        default: launch_thin<R9VX_SCHEME_IQ3_S>(a, nr, nc, stream); break;
+        }
+        const int e = (int)hipGetLastError();
+        if (e) return e;
     }
-    switch (p.scheme) {
-    case R9VX_SCHEME_Q4_K: launch_thin<R9VX_SCHEME_Q4_K>(a, nr, nc, stream); break;
-    case R9VX_SCHEME_IQ4_XS: launch_thin<R9VX_SCHEME_IQ4_XS>(a, nr, nc, stream); break;
-    case R9VX_SCHEME_Q6_K: launch_thin<R9VX_SCHEME_Q6_K>(a, nr, nc, stream); break;
-    case R9VX_SCHEME_Q8_0: launch_thin<R9VX_SCHEME_Q8_0>(a, nr, nc, stream); break;
-    default: launch_thin<R9VX_SCHEME_IQ3_S>(a, nr, nc, stream); break;
-    }
-    return (int)hipGetLastError();
+    return 0;
 }

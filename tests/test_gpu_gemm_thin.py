@@ -93,3 +93,16 @@ def test_thin_tiles_under_a_captured_graph():
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(y, want)
+
+
+def test_thin_rows_past_one_launch():
+    """More rows than one launch takes (2^20): the rows beside the cut and the
+    last ones have the bits of a launch of their own, bias and residual."""
+    m, n, k = (1 << 20) + 45, 40, 256
+    _, w, _ = _weight(O.Q4_K, 9870, n, k)
+    x = torch.randn((m, k), generator=torch.Generator(device="cuda").manual_seed(9871), device="cuda", dtype=torch.bfloat16)
+    res = torch.randn((m, n), generator=torch.Generator(device="cuda").manual_seed(9872), device="cuda")
+    y = ffi.matmul(w, O.Q4_K, n, k, x, residual=res)
+    for rows in (slice(0, 64), slice((1 << 20) - 40, (1 << 20) + 40), slice(m - 33, m)):
+        alone = ffi.matmul(w, O.Q4_K, n, k, x[rows].contiguous(), residual=res[rows].contiguous())
+        assert torch.equal(y[rows], alone), rows

@@ -38,3 +38,16 @@ def test_router_launches(runtime, e, scoring, line):
     last, past = kernels(runtime, [("route", dict(t=t, e=e, k=8, scoring=scoring)) for t in (line, line + 1)])
     assert len(last) == 1 and last[0].startswith("route_small_kernel")
     assert [k.split("<")[0] for k in past] == ["clear_status_kernel", "route_check_kernel", "route_kernel"]
+
+
+@pytest.mark.parametrize("m,n,k", [((1 << 24) + 7, 64, 256), (1 << 24, 1, 256), ((1 << 20) + 1, 33, 512), (1 << 20, 64, 256)])
+def test_prefill_rows_within_the_launch_limits(runtime, m, n, k):
+    """Row counts past 2^32 / 256: every row converted once and in a tile, in
+    launches that HIP accepts."""
+    (rc, msg, launches), = launch_record.record(runtime, [("matmul", dict(scheme=ffi.Q4_K, m=m, n=n, k=k))])
+    assert rc == 0, msg
+    thin = [(name, g) for name, g, _ in launches if name.startswith("gemm_thin_kernel")]
+    assert len(thin) == -(-m // (1 << 20)) and len(launches) == 2 * len(thin)
+    assert sum(g[0] for name, g, _ in launches if "x_to_f16_thin" in name) == m
+    tiles = [32 * int(name.split("<")[1].split(",")[1]) * g[1] for name, g in thin]
+    assert tiles[:-1] == [1 << 20] * (len(thin) - 1) and 0 <= sum(tiles) - m < 256
