@@ -273,8 +273,9 @@ uint64_t gemm3_cost(const GemmArgs &a, uint32_t wgs, uint32_t cus) {
 struct ThinShape {
     uint32_t nr, nc, ns, load; /* ns + load x (the share of the CUs at work) */
 };
-constexpr ThinShape kThinShapes[] = {{1, 1, 500, 0},   {2, 1, 600, 0},    {4, 1, 900, 0},    {1, 2, 930, 0},
-                                     {2, 2, 1060, 0}, {4, 2, 900, 830}, {8, 2, 1300, 1500}};
+#define R9VX_THIN_SHAPE(NR, NC, NS, LOAD) {NR, NC, NS, LOAD},
+constexpr ThinShape kThinShapes[] = {R9VX_THIN_SHAPES(R9VX_THIN_SHAPE)};
+#undef R9VX_THIN_SHAPE
 
 /* One round of `wgs` workgroups of nc column tiles and `tiles` active row tiles. */
 uint64_t thin_round(uint32_t nc, uint32_t tiles, uint64_t wgs, uint32_t cus) {

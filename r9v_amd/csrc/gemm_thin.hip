@@ -330,18 +330,16 @@ __global__ __launch_bounds__(64 * (NR + kThinDec)) void gemm_thin_kernel(ThinArg
 constexpr uint32_t kThinMaxRows = 1u << 20;
 
 template <int SCHEME>
-void launch_thin(const ThinArgs &a, uint32_t nr, uint32_t nc, hipStream_t s) {
+int launch_thin(const ThinArgs &a, uint32_t nr, uint32_t nc, hipStream_t s) {
     const dim3 grid((a.n + 32 * nc - 1) / (32 * nc), (a.m + 32 * nr - 1) / (32 * nr)), block(64 * (nr + kThinDec));
-#define R9VX_THIN(NR, NC) \
-    if (nr == NR && nc == NC) hipLaunchKernelGGL((gemm_thin_kernel<SCHEME, NR, NC>), grid, block, 0, s, a);
-    R9VX_THIN(1, 1)
-    R9VX_THIN(2, 1)
-    R9VX_THIN(4, 1)
-    R9VX_THIN(1, 2)
-    R9VX_THIN(2, 2)
-    R9VX_THIN(4, 2)
-    R9VX_THIN(8, 2)
+#define R9VX_THIN(NR, NC, NS, LOAD)                                                      \
+    if (nr == NR && nc == NC) {                                                          \
+        hipLaunchKernelGGL((gemm_thin_kernel<SCHEME, NR, NC>), grid, block, 0, s, a);    \
+        return (int)hipGetLastError();                                                   \
+    }
+    R9VX_THIN_SHAPES(R9VX_THIN)
 #undef R9VX_THIN
+    return (int)hipErrorInvalidValue;
 }
 
 void launch_x16(uint32_t order, const uint16_t *x, uint32_t m, uint32_t k, _Float16 *x16, float *scale, hipStream_t s) {
@@ -377,14 +375,15 @@ int r9vx_launch_gemm_thin(const r9vx_gemm_problem &p, uint32_t nr, uint32_t nc, 
         a.residual = p.residual ? p.residual + (size_t)r0 * p.n : nullptr;
         a.y = reinterpret_cast<uint8_t *>(p.y) + (size_t)r0 * p.n * (a.y_bf16 ? 2 : 4);
         launch_x16(r9vx_group_order(p.scheme), p.x + (size_t)r0 * p.k, a.m, p.k, x16 + (size_t)r0 * p.k, scale + r0, stream);
+        int e = (int)hipGetLastError();
+        if (e) return e;
         switch (p.scheme) {
-        case R9VX_SCHEME_Q4_K: launch_thin<R9VX_SCHEME_Q4_K>(a, nr, nc, stream); break;
-        case R9VX_SCHEME_IQ4_XS: launch_thin<R9VX_SCHEME_IQ4_XS>(a, nr, nc, stream); break;
-        case R9VX_SCHEME_Q6_K: launch_thin<R9VX_SCHEME_Q6_K>(a, nr, nc, stream); break;
-        case R9VX_SCHEME_Q8_0: launch_thin<R9VX_SCHEME_Q8_0>(a, nr, nc, stream); break;
-        default: launch_thin<R9VX_SCHEME_IQ3_S>(a, nr, nc, stream); break;
+        case R9VX_SCHEME_Q4_K: e = launch_thin<R9VX_SCHEME_Q4_K>(a, nr, nc, stream); break;
+        case R9VX_SCHEME_IQ4_XS: e = launch_thin<R9VX_SCHEME_IQ4_XS>(a, nr, nc, stream); break;
+        case R9VX_SCHEME_Q6_K: e = launch_thin<R9VX_SCHEME_Q6_K>(a, nr, nc, stream); break;
+        case R9VX_SCHEME_Q8_0: e = launch_thin<R9VX_SCHEME_Q8_0>(a, nr, nc, stream); break;
+        default: e = launch_thin<R9VX_SCHEME_IQ3_S>(a, nr, nc, stream); break;
         }
-        const int e = (int)hipGetLastError();
         if (e) return e;
     }
     return 0;

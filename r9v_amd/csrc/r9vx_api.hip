@@ -175,14 +175,17 @@ uint64_t r9vx_matmul_static_flops(const r9vx_matmul_static *st, uint32_t m) {
     return (st->epilogue == R9VX_EPILOGUE_SWIGLU ? 4ull : 2ull) * m * st->n * st->k;
 }
 
-int r9vx_matmul_launch(const r9vx_matmul_static *st, const r9vx_matmul_args *a,
-                       r9vx_stream_t stream) {
+/* nr, nc: the thin tiles' shape (0, 0: the kernel by the size rule) */
+static int matmul_launch(const char *op, const r9vx_matmul_static *st, const r9vx_matmul_args *a, uint32_t nr,
+                         uint32_t nc, r9vx_stream_t stream) {
     Problems pr;
     if (!st || !a) {
         pr.add(R9VX_ERR_NULL, "static and args must be non-NULL");
-        return pr.finish("matmul");
+        return pr.finish(op);
     }
     check_matmul_static(st, pr);
+    if (nr && (st->in_dtype != R9VX_DTYPE_BF16 || st->m_bucket <= 8))
+        pr.add(R9VX_ERR_UNSUPPORTED, "the thin tiles take bf16 activations and m_bucket > 8");
     if (a->m > st->m_bucket)
         pr.add(R9VX_ERR_INVALID, "m=%u exceeds m_bucket=%u", a->m, st->m_bucket);
     if (a->m > 0) {
@@ -212,7 +215,7 @@ int r9vx_matmul_launch(const r9vx_matmul_static *st, const r9vx_matmul_args *a,
         else if ((uintptr_t)a->workspace & 255u)
             pr.add(R9VX_ERR_ALIGN, "workspace must be 256-byte aligned");
     }
-    int rc = pr.finish("matmul");
+    int rc = pr.finish(op);
     if (rc || a->m == 0) return rc;
 
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
@@ -239,7 +242,7 @@ int r9vx_matmul_launch(const r9vx_matmul_static *st, const r9vx_matmul_args *a,
         g.scheme = st->w_scheme;
         g.y_dtype = st->out_dtype;
         g.epilogue = st->epilogue;
-        return hip_status("matmul", r9vx_launch_gemm(g, s));
+        return hip_status(op, nr ? r9vx_launch_gemm_thin(g, nr, nc, s) : r9vx_launch_gemm(g, s));
     }
     /* GEMV, eight activation rows per launch. */
     const uint32_t xe = st->in_dtype == R9VX_DTYPE_F32 ? 4 : 2;
@@ -262,9 +265,23 @@ int r9vx_matmul_launch(const r9vx_matmul_static *st, const r9vx_matmul_args *a,
         p.w_row_stride = w_row;
         p.x_row_stride = st->k;
         int e = r9vx_launch_gemv(p, s);
-        if (e) return hip_status("matmul", e);
+        if (e) return hip_status(op, e);
     }
     return R9VX_OK;
+}
+
+int r9vx_matmul_launch(const r9vx_matmul_static *st, const r9vx_matmul_args *a, r9vx_stream_t stream) {
+    return matmul_launch("matmul", st, a, 0, 0, stream);
+}
+
+int r9vx_probe_matmul_thin_launch(const r9vx_matmul_static *st, const r9vx_matmul_args *a, uint32_t nr, uint32_t nc,
+                                  r9vx_stream_t stream) {
+    if (nr == 0 || nc == 0) {
+        Problems pr;
+        pr.add(R9VX_ERR_INVALID, "nr=%u, nc=%u: no thin tile is empty", nr, nc);
+        return pr.finish("probe_matmul_thin");
+    }
+    return matmul_launch("probe_matmul_thin", st, a, nr, nc, stream);
 }
 
 /* ----------------------------------------------------------- weights/decode */

@@ -117,7 +117,11 @@ size_t r9vx_gemm_workspace_bytes(uint32_t m_bucket, uint32_t k);
 size_t r9vx_gemm_x16_bytes(uint32_t m, uint32_t k);
 int r9vx_launch_gemm(const r9vx_gemm_problem &p, hipStream_t stream);
 /* The thin-tile form (gemm_thin.hip): nr row tiles of 32 rows and nc column
- * tiles of 32 columns per workgroup.  Output bits equal r9vx_launch_gemm's. */
+ * tiles of 32 columns per workgroup.  Output bits equal r9vx_launch_gemm's.
+ * Shapes that do not exist are refused.  They are (nr, nc, ns, load): the last
+ * two are the cost of a super-block in the size rule (gemm.hip, thin_plan). */
+#define R9VX_THIN_SHAPES(X) \
+    X(1, 1, 500, 0) X(2, 1, 600, 0) X(4, 1, 900, 0) X(1, 2, 930, 0) X(2, 2, 1060, 0) X(4, 2, 900, 830) X(8, 2, 1300, 1500)
 int r9vx_launch_gemm_thin(const r9vx_gemm_problem &p, uint32_t nr, uint32_t nc, hipStream_t stream);
 /* Compute units of the current device (cached per device; 256 if the query fails). */
 uint32_t r9vx_device_cus();

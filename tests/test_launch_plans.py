@@ -51,3 +51,22 @@ def test_prefill_rows_within_the_launch_limits(runtime, m, n, k):
     assert sum(g[0] for name, g, _ in launches if "x_to_f16_thin" in name) == m
     tiles = [32 * int(name.split("<")[1].split(",")[1]) * g[1] for name, g in thin]
     assert tiles[:-1] == [1 << 20] * (len(thin) - 1) and 0 <= sum(tiles) - m < 256
+
+
+THIN_SHAPES = [(1, 1), (2, 1), (4, 1), (1, 2), (2, 2), (4, 2), (8, 2)]
+
+
+@pytest.mark.parametrize("scheme", [ffi.Q4_K, ffi.IQ4_XS, ffi.Q6_K, ffi.Q8_0, ffi.IQ3_S])
+def test_thin_shapes_launch_or_are_refused(runtime, scheme):
+    """Every pair of row and column tiles runs its kernel or is an error: none
+    returns 0 with nothing launched."""
+    pairs = [(nr, nc) for nr in (1, 2, 3, 4, 6, 8, 16) for nc in (1, 2, 4)]
+    out = launch_record.record(runtime, [("matmul", dict(scheme=scheme, m=300, n=500, k=512, thin=p)) for p in pairs])
+    for (nr, nc), (rc, _, launches) in zip(pairs, out):
+        ran = [k for k, _, _ in launches if k.startswith("gemm")]
+        assert ran == ([f"gemm_thin_kernel<{scheme}, {nr}, {nc}>"] if (nr, nc) in THIN_SHAPES else []), (nr, nc)
+        assert (rc == 0) == bool(ran), (nr, nc, rc)
+    # and the decode bucket and f32 activations have none
+    for kw in (dict(m=8), dict(m=300, x_f32=True), dict(m=300, scheme=ffi.Q4_K, x_f32=True)):
+        call = dict(dict(scheme=scheme, n=500, k=512, thin=(1, 1)), **kw)
+        assert launch_record.record(runtime, [("matmul", call)])[0][0] < 0
