@@ -253,21 +253,43 @@ uint32_t plan_chunks(GemmArgs &a, uint32_t cus) {
 }
 
 /* Which kernel: both run in rounds of one workgroup per CU, and a workgroup's
- * time per super-block (256 K) follows from its shape, so the launch with the
- * least sum over its rounds is taken.  The constants are nanoseconds measured
- * on Q4_K at k = 4096 (launch times less 8 us, over 16 super-blocks; the other
- * schemes' are within 20% in the same order).  A 256-column workgroup's step
- * costs 2900 whatever its rows and 680 per row tile.  A thin one's follows its
+ * time per super-block (256 K) follows from its shape and the scheme's decode, so
+ * the launch with the least sum over its rounds is taken.  The constants are
+ * nanoseconds, fitted to 4660 sizes timed with the 256-column tiles and every
+ * thin shape near the best (all five schemes, k of 256 to 14336, n of 512 to
+ * 16384, m of 9 to 4096): 20 of them take a kernel that is over 3% slower than
+ * the 256-column tiles, by at most 12% (from k = 1024 11, 8%).  Constants of
+ * Q4_K at k = 4096 and m up to 1024 alone left 145, up to 41%.
+ *
+ * A 256-column workgroup decodes at a time of its own (base, 500 per row tile)
+ * until its MFMAs (710 per row tile) take longer.  A thin one's time follows its
  * active row tiles and, where those read enough activations to fill the L2's
- * bandwidth, how many of the CUs work beside it: 64 columns x 8 row tiles
- * 2100 on 160 CUs, 2850 on 256.  k = 4096, us, 256-column tiles / thin ones:
- *   n = 4096:  m = 32: 61 / 16, 128: 60 / 20, 512: 62 / 36, 1024: 71 / 54
- *   n = 14336: m = 32: 62 / 25, 128: 63 / 32, 256: 71 / 48, 512: 104 / 85
- * and Q6_K n = 2048, k = 14336, m = 64: 254 / 44.  Up to 4 row tiles a
- * workgroup alone: n = 4096 m = 777 55 us (with 8: 48), 1024 65 (54). */
-uint64_t gemm3_cost(const GemmArgs &a, uint32_t wgs, uint32_t cus) {
+ * bandwidth, how many of the CUs work beside it.  Its launch adds, per row, what
+ * its conversion of the activations costs more (it writes 16 bytes at a time)
+ * and, per round, a workgroup's entry.  k = 4096, us, 256-column tiles / thin:
+ *   Q4_K n = 4096:  m = 32: 61 / 16, 128: 60 / 20, 512: 62 / 36, 1024: 71 / 54
+ *   Q4_K n = 14336: m = 32: 62 / 25, 128: 63 / 32, 256: 71 / 48, 512: 104 / 85
+ * and where the line lies:
+ *   Q4_K n = 3072 m = 1300: 69 / 67, 1600: 76 / 80; n = 2048 m = 2048: 72 / 60,
+ *   2600: 82 / 91, 4096: 101 / 116; n = 512 m = 4096: 66 / 75
+ *   IQ3_S n = 2048 m = 4096: 118 / 118; n = 4096 m = 2048: 111 / 100 */
+struct SchemeCost {
+    uint32_t base, thin; /* ns of a 256-column step's decode; the thin times in % */
+};
+SchemeCost scheme_cost(uint32_t scheme) {
+    switch (scheme) {
+    case R9VX_SCHEME_Q4_K: return {2850, 100};
+    case R9VX_SCHEME_IQ4_XS: return {3800, 104};
+    case R9VX_SCHEME_Q6_K: return {3700, 102};
+    case R9VX_SCHEME_Q8_0: return {3350, 98};
+    default: return {5150, 116};
+    }
+}
+
+uint64_t gemm3_cost(const GemmArgs &a, uint32_t scheme, uint32_t wgs, uint32_t cus) {
     const uint32_t per = (a.rt + a.nlo - 1) / a.nlo; /* row tiles of the largest chunk */
-    return (uint64_t)((wgs + cus - 1) / cus) * (2900u + 680u * per);
+    const uint32_t decode = scheme_cost(scheme).base + 500u * per, mfma = 2250u + 710u * per;
+    return (uint64_t)((wgs + cus - 1) / cus) * (decode > mfma ? decode : mfma) * (a.k / 256);
 }
 
 struct ThinShape {
@@ -284,24 +306,25 @@ uint64_t thin_round(uint32_t nc, uint32_t tiles, uint64_t wgs, uint32_t cus) {
     return ~0u;
 }
 
-uint64_t thin_plan(uint32_t m, uint32_t n, uint32_t cus, uint32_t &nr, uint32_t &nc) {
-    uint64_t best = ~0ull;
+uint64_t thin_plan(uint32_t m, uint32_t n, uint32_t k, uint32_t scheme, uint32_t cus, uint32_t &nr, uint32_t &nc) {
+    uint64_t best = ~0ull, best_rounds = 0;
     const uint32_t tiles = (m + 31) / 32;
     for (const auto &s : kThinShapes) {
         const uint64_t strips = (n + 32 * s.nc - 1) / (32 * s.nc);
         /* workgroups of nr row tiles, dealt first, then one of the rest per strip */
         const uint64_t full = strips * (tiles / s.nr), rem = full % cus;
         uint64_t rest = tiles % s.nr ? strips : 0;
-        uint64_t cost = full / cus * thin_round(s.nc, s.nr, cus, cus);
+        uint64_t cost = full / cus * thin_round(s.nc, s.nr, cus, cus), rounds = full / cus;
         if (rem) { /* the last round of full ones, and what fits beside it */
             const uint64_t beside = rest < cus - rem ? rest : cus - rem;
             cost += thin_round(s.nc, s.nr, rem + beside, cus);
             rest -= beside;
+            ++rounds;
         }
-        for (; rest; rest -= rest < cus ? rest : cus) cost += thin_round(s.nc, tiles % s.nr, rest, cus);
-        if (cost < best) best = cost, nr = s.nr, nc = s.nc;
+        for (; rest; rest -= rest < cus ? rest : cus, ++rounds) cost += thin_round(s.nc, tiles % s.nr, rest, cus);
+        if (cost < best) best = cost, best_rounds = rounds, nr = s.nr, nc = s.nc;
     }
-    return best;
+    return (best * scheme_cost(scheme).thin / 100 + 9 * (uint64_t)m / 20) * (k / 256) + 500 * best_rounds + 250;
 }
 
 }  // namespace
@@ -374,7 +397,8 @@ int r9vx_launch_gemm(const r9vx_gemm_problem &p, hipStream_t stream) {
         GemmArgs whole = a;
         const uint32_t wgs = plan_chunks(whole, cus);
         uint32_t nr = 0, nc = 0;
-        if (thin_plan(p.m, p.n, cus, nr, nc) < gemm3_cost(whole, wgs, cus)) return r9vx_launch_gemm_thin(p, nr, nc, stream);
+        if (thin_plan(p.m, p.n, p.k, p.scheme, cus, nr, nc) < gemm3_cost(whole, p.scheme, wgs, cus))
+            return r9vx_launch_gemm_thin(p, nr, nc, stream);
     }
     const int rc = r9vx_launch_x_to_f16(p.x, p.m, p.k, x16, scale, r9vx_group_order(p.scheme), stream);
     if (rc) return rc;

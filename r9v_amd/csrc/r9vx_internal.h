@@ -121,7 +121,8 @@ int r9vx_launch_gemm(const r9vx_gemm_problem &p, hipStream_t stream);
  * Shapes that do not exist are refused.  They are (nr, nc, ns, load): the last
  * two are the cost of a super-block in the size rule (gemm.hip, thin_plan). */
 #define R9VX_THIN_SHAPES(X) \
-    X(1, 1, 500, 0) X(2, 1, 600, 0) X(4, 1, 900, 0) X(1, 2, 930, 0) X(2, 2, 1060, 0) X(4, 2, 900, 830) X(8, 2, 1300, 1500)
+    X(1, 1, 780, 0) X(2, 1, 900, 0) X(4, 1, 1040, 0) X(1, 2, 1090, 450) X(2, 2, 1280, 50) X(4, 2, 960, 730) \
+    X(8, 2, 1080, 1250)
 int r9vx_launch_gemm_thin(const r9vx_gemm_problem &p, uint32_t nr, uint32_t nc, hipStream_t stream);
 /* Compute units of the current device (cached per device; 256 if the query fails). */
 uint32_t r9vx_device_cus();

@@ -102,7 +102,7 @@ def test_thin_rows_past_one_launch():
     _, w, _ = _weight(O.Q4_K, 9870, n, k)
     x = torch.randn((m, k), generator=torch.Generator(device="cuda").manual_seed(9871), device="cuda", dtype=torch.bfloat16)
     res = torch.randn((m, n), generator=torch.Generator(device="cuda").manual_seed(9872), device="cuda")
-    y = ffi.matmul(w, O.Q4_K, n, k, x, residual=res)
+    y = ffi.probe_matmul_thin(w, O.Q4_K, n, k, x, 8, 2, residual=res)
     for rows in (slice(0, 64), slice((1 << 20) - 40, (1 << 20) + 40), slice(m - 33, m)):
         alone = ffi.matmul(w, O.Q4_K, n, k, x[rows].contiguous(), residual=res[rows].contiguous())
         assert torch.equal(y[rows], alone), rows

@@ -42,10 +42,13 @@ def test_router_launches(runtime, e, scoring, line):
 
 @pytest.mark.parametrize("m,n,k", [((1 << 24) + 7, 64, 256), (1 << 24, 1, 256), ((1 << 20) + 1, 33, 512), (1 << 20, 64, 256)])
 def test_prefill_rows_within_the_launch_limits(runtime, m, n, k):
-    """Row counts past 2^32 / 256: every row converted once and in a tile, in
-    launches that HIP accepts."""
-    (rc, msg, launches), = launch_record.record(runtime, [("matmul", dict(scheme=ffi.Q4_K, m=m, n=n, k=k))])
+    """Row counts past 2^32 / 256: launches that HIP accepts, and on the thin
+    tiles every row converted once and in a tile."""
+    call = dict(scheme=ffi.Q4_K, m=m, n=n, k=k)
+    (rc, msg, _), (thin_rc, thin_msg, launches) = launch_record.record(
+        runtime, [("matmul", call), ("matmul", dict(call, thin=(8, 2)))])
     assert rc == 0, msg
+    assert thin_rc == 0, thin_msg
     thin = [(name, g) for name, g, _ in launches if name.startswith("gemm_thin_kernel")]
     assert len(thin) == -(-m // (1 << 20)) and len(launches) == 2 * len(thin)
     assert sum(g[0] for name, g, _ in launches if "x_to_f16_thin" in name) == m
@@ -70,3 +73,19 @@ def test_thin_shapes_launch_or_are_refused(runtime, scheme):
     for kw in (dict(m=8), dict(m=300, x_f32=True), dict(m=300, scheme=ffi.Q4_K, x_f32=True)):
         call = dict(dict(scheme=scheme, n=500, k=512, thin=(1, 1)), **kw)
         assert launch_record.record(runtime, [("matmul", call)])[0][0] < 0
+
+
+# sizes beside the line between the two prefill kernels (256 compute units), each
+# with the kernel that was measured the faster there (gemm.hip, gemm3_cost)
+PREFILL_SIDES = [(ffi.Q4_K, 32, 14336, 4096, "thin"), (ffi.Q4_K, 777, 4096, 4096, "thin"),
+                 (ffi.Q4_K, 2048, 2048, 4096, "thin"), (ffi.Q4_K, 2600, 2048, 4096, "gemm3"),
+                 (ffi.Q4_K, 4096, 2048, 4096, "gemm3"), (ffi.Q4_K, 1600, 3072, 4096, "gemm3"),
+                 (ffi.Q8_0, 4096, 2048, 14336, "gemm3"), (ffi.Q4_K, 4096, 512, 4096, "gemm3"),
+                 (ffi.IQ3_S, 2048, 4096, 4096, "thin"), (ffi.Q6_K, 1600, 3072, 256, "gemm3"),
+                 (ffi.Q4_K, 2048, 14336, 4096, "gemm3"), (ffi.Q6_K, 57, 4096, 14336, "thin")]
+
+
+@pytest.mark.parametrize("scheme,m,n,k,kernel", PREFILL_SIDES)
+def test_prefill_kernel_by_size(runtime, scheme, m, n, k, kernel):
+    (names,) = kernels(runtime, [("matmul", dict(scheme=scheme, m=m, n=n, k=k))])
+    assert names[-1].startswith({"thin": "gemm_thin_kernel", "gemm3": "gemm3_kernel"}[kernel]), names
