@@ -111,3 +111,24 @@ def test_infinite_last_block_is_not_nan(scheme, n, k, m, swiglu, x_f32):
     x = torch.ones((m, k), dtype=torch.float32 if x_f32 else torch.bfloat16, device="cuda")
     y = ffi.matmul(w, scheme, n, k, x, w_scales=sc, swiglu=swiglu)
     assert bool((y == float("inf")).all())
+
+
+@pytest.mark.parametrize("scheme", [O.Q4_K, O.IQ3_S])
+@pytest.mark.parametrize("n,k,swiglu", [(16384, 2304, False), (16391, 2816, False), (32768, 768, False),
+                                        (5120, 2304, True), (5133, 4352, True), (10240, 1280, True)])
+def test_many_ragged_rows_take_fewer_lanes(scheme, n, k, swiglu):
+    """From the lines where a row's idle lanes cost more than their latency: the
+    oracle's values at sampled rows, and the same bits in every bucket."""
+    rows = 2 * n if swiglu else n
+    wire, w, sc = _weight(scheme, 9990 + k, rows, k)
+    x, xd = _x(9991 + k, 8, k)
+    cols = np.r_[0:9, n // 2 - 5:n // 2 + 5, n - 9:n]
+    some = np.ascontiguousarray(wire.reshape(rows, -1)[np.r_[cols, cols + n] if swiglu else cols])
+    want = O.matmul(scheme, some, len(some), k, x, O.BF16)
+    if swiglu:
+        g, u = want[:, :len(cols)].astype(np.float64), want[:, len(cols):].astype(np.float64)
+        want = (g / (1.0 + np.exp(-g)) * u).astype(np.float32)
+    whole = ffi.matmul(w, scheme, n, k, xd, w_scales=sc, swiglu=swiglu)
+    check_close(whole.cpu().numpy()[:, cols], want, f"{scheme} n={n} k={k}")
+    for m in (1, 2, 4, 5):
+        assert torch.equal(ffi.matmul(w, scheme, n, k, xd[:m], w_scales=sc, swiglu=swiglu), whole[:m]), f"m={m}"

@@ -89,3 +89,22 @@ PREFILL_SIDES = [(ffi.Q4_K, 32, 14336, 4096, "thin"), (ffi.Q4_K, 777, 4096, 4096
 def test_prefill_kernel_by_size(runtime, scheme, m, n, k, kernel):
     (names,) = kernels(runtime, [("matmul", dict(scheme=scheme, m=m, n=n, k=k))])
     assert names[-1].startswith({"thin": "gemm_thin_kernel", "gemm3": "gemm3_kernel"}[kernel]), names
+
+
+# n, K, gated: the first sizes at which a ragged row is read by fewer than 64 lanes
+FEWER_LANES = [(16384, 2304, False), (16384, 6400, False), (32768, 768, False), (5120, 2304, True), (10240, 1280, True),
+               (24576, 768, True)]
+
+
+@pytest.mark.parametrize("n,k,swiglu", FEWER_LANES)
+@pytest.mark.parametrize("m", [1, 3, 8])
+def test_lanes_of_many_ragged_rows(runtime, n, k, swiglu, m):
+    """A wave takes several rows from the line on (fewer waves, or the kernel
+    of any number of lanes), for every m alike; 1024 SIMDs."""
+    def launch(rows):
+        (out,) = launch_record.record(runtime, [("matmul", dict(scheme=ffi.Q4_K, m=m, n=rows, k=k, m_bucket=8,
+                                                                epilogue=3 if swiglu else 0))])
+        (name, g, b), = out[2]
+        return name, g[0] * b[0] // 64
+    (name, waves), (below, waves_below) = launch(n), launch(n - 1)
+    assert name != below or waves < 0.9 * waves_below
