@@ -553,6 +553,31 @@ __global__ __launch_bounds__(waves_for(M) * 64) void gemv_gated_kernel(GemvArgs 
  * n = 2816, K = 2048, m = 1: 4.44 against 4.76 us). */
 constexpr uint32_t kGatedMaxSteps = 16;
 
+/* Where it is the faster one: what it saves per row (x again) against its two
+ * waves a SIMD, fewer where its registers are many.  Streaming / one-shot at n
+ * of 8192 to 24000 (K = 2048 and 1792 with one chunk a lane, 4096 and 3840 with two):
+ *            m = 1        2            3            4
+ *   two Q4_K 0.89 - 0.97  0.88 - 0.98  0.59 - 0.73  0.67 - 0.79
+ *     IQ4_XS 1.02 - 1.10  0.90 - 1.04  0.83 - 0.92  0.80 - 0.91
+ *       Q6_K 0.85 - 0.95  0.93 - 1.02  0.66 - 0.90  0.74 - 0.88
+ *       Q8_0 1.02 - 1.08  0.90 - 0.97  0.91 - 1.03  0.70 - 0.83
+ *      IQ3_S 0.93 - 1.01  0.92 - 0.98  0.80 - 0.86  0.78 - 0.82
+ *   one Q4_K 1.06 - 1.22  0.98 - 1.11  1.00 - 1.10  1.01 - 1.08
+ *     IQ4_XS 1.11 - 1.31  0.98 - 1.12  0.98 - 1.04  0.92 - 0.99
+ *       Q6_K 1.03 - 1.20  0.78 - 1.02  1.06 - 1.19  0.84 - 0.90
+ *       Q8_0 1.05 - 1.17  1.02 - 1.09  0.88 - 0.99  0.88 - 1.00
+ *      IQ3_S 1.01 - 1.06  0.91 - 0.96  0.84 - 0.88  0.80 - 0.84 */
+constexpr bool gated_streams(int scheme, int spl, int m) {
+    if (spl == 2) return m > 1 || (scheme != R9VX_SCHEME_IQ4_XS && scheme != R9VX_SCHEME_Q8_0);
+    switch (scheme) {
+    case R9VX_SCHEME_IQ4_XS: return m == 4;
+    case R9VX_SCHEME_Q6_K: return m == 2 || m == 4;
+    case R9VX_SCHEME_Q8_0: return m >= 3;
+    case R9VX_SCHEME_IQ3_S: return m >= 2;
+    default: return false;
+    }
+}
+
 template <int SCHEME, int M, int SPL, bool RAG>
 __global__ __launch_bounds__(256) void gemv_gated_stream_kernel(GemvArgs a, uint32_t steps) {
     using Pay = typename std::conditional<pay2_scheme(SCHEME), Payload2, r9vx_u32x4>::type;
@@ -653,14 +678,16 @@ __global__ __launch_bounds__(256) void gemv_gated_stream_kernel(GemvArgs a, uint
     }
 }
 
+uint32_t device_simds();
+
 template <int SCHEME, int SPL, int MM>
 int launch_gated_stream(const GemvArgs &a, uint32_t m, uint32_t simds, hipStream_t s) {
     if constexpr (MM == 0) {
         return (int)hipErrorInvalidValue;
     } else {
         if (m != MM) return launch_gated_stream<SCHEME, SPL, MM - 1>(a, m, simds, s);
+        if constexpr (!gated_streams(SCHEME, SPL, MM)) return (int)hipErrorInvalidValue;
         uint32_t waves = kStreamWavesPerSimd * simds;
-        if (waves > a.n) waves = a.n;
         if ((a.n + waves - 1) / waves > kGatedMaxSteps) waves = (a.n + kGatedMaxSteps - 1) / kGatedMaxSteps;
         const uint32_t wgs = (waves + 3) / 4, steps = (a.n + wgs * 4 - 1) / (wgs * 4);
         if (a.ragged)
@@ -688,8 +715,6 @@ int launch_gated(const GemvArgs &a, uint32_t m, uint32_t groups, hipStream_t s) 
     }
 }
 
-uint32_t device_simds();
-
 template <int SCHEME>
 int launch_gated_scheme(const GemvArgs &a, uint32_t m, int spl, uint32_t g, hipStream_t s) {
     /* IQ3_S carries a wider chunk (payload, signs and side word): two row
@@ -698,7 +723,7 @@ int launch_gated_scheme(const GemvArgs &a, uint32_t m, int spl, uint32_t g, hipS
     constexpr int kTwoPairMaxM = SCHEME == R9VX_SCHEME_IQ3_S ? 5 : 8;
     if (a.lpr_log2 == 6 && a.nseg == 1 && m <= 4) {
         const uint32_t simds = device_simds();
-        if (a.n >= 8 * simds)
+        if (a.n >= 8 * simds && gated_streams(SCHEME, spl, (int)m))
             return spl == 2 ? launch_gated_stream<SCHEME, 2, 4>(a, m, simds, s) : launch_gated_stream<SCHEME, 1, 4>(a, m, simds, s);
     }
     if (a.n >= 8 * device_simds() && (int)m <= kTwoPairMaxM)

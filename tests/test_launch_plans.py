@@ -108,3 +108,16 @@ def test_lanes_of_many_ragged_rows(runtime, n, k, swiglu, m):
         return name, g[0] * b[0] // 64
     (name, waves), (below, waves_below) = launch(n), launch(n - 1)
     assert name != below or waves < 0.9 * waves_below
+
+
+@pytest.mark.parametrize("scheme,k,streams", [(ffi.Q4_K, 2048, ()), (ffi.IQ4_XS, 2048, (4,)), (ffi.Q6_K, 2048, (2, 4)),
+                                              (ffi.Q8_0, 2048, (3, 4)), (ffi.IQ3_S, 2048, (2, 3, 4)),
+                                              (ffi.Q4_K, 4096, (1, 2, 3, 4)), (ffi.IQ4_XS, 4096, (2, 3, 4)),
+                                              (ffi.Q6_K, 4096, (1, 2, 3, 4)), (ffi.Q8_0, 4096, (2, 3, 4)),
+                                              (ffi.IQ3_S, 4096, (1, 2, 3, 4))])
+def test_gated_streaming_where_it_is_faster(runtime, scheme, k, streams):
+    """n = 14336, the gated epilogue: the streaming kernel for the row counts at
+    which it was measured the faster, the one-shot kernel elsewhere (the same bits)."""
+    names = kernels(runtime, [("matmul", dict(scheme=scheme, m=m, n=14336, k=k, epilogue=3)) for m in (1, 2, 3, 4, 5)])
+    for m, (name,) in zip((1, 2, 3, 4, 5), names):
+        assert name.startswith("gemv_gated_stream_kernel" if m in streams else "gemv_gated_kernel"), (m, name)
