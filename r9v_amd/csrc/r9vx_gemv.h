@@ -419,12 +419,17 @@ int launch_stream(const GemvArgs &a, uint32_t simds, hipStream_t s) {
  * one below (measured, Q4_K, graph replay: n = 14336, K = 4096, M = 4:
  * 39.2 us at two against 49.1 at one and 64.9 at three; n = 2816, K = 2048,
  * M = 8: 11.5 us at one against 21.3 at two). */
+/* Waves of a workgroup, at most: IQ3_S rows share the codebook's table (4 KiB to
+ * build) between four from 2 x SIMDs waves on (m = 8, n = 16384, K = 1792 55.6 ->
+ * 45.1 us; n = 768, K = 512 6.1 / 5.3, so not below). */
+constexpr int gated_waves_for(int scheme, int m) { return scheme == R9VX_SCHEME_IQ3_S && m >= 3 ? 4 : waves_for(m); }
+
 template <int SCHEME, int M, int SPL, int PAIRS, bool RAG>
-__global__ __launch_bounds__(waves_for(M) * 64) void gemv_gated_kernel(GemvArgs a) {
-    constexpr int kRows = PAIRS, kWaves = waves_for(M);
+__global__ __launch_bounds__(gated_waves_for(SCHEME, M) * 64) void gemv_gated_kernel(GemvArgs a) {
+    constexpr int kRows = PAIRS;
     __shared__ __attribute__((aligned(16))) uint32_t lut[lut_words(SCHEME)];
     const uint32_t lane = threadIdx.x & 63;
-    const uint32_t wave = blockIdx.x * kWaves + (threadIdx.x >> 6);
+    const uint32_t wave = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
     const uint32_t lprl = a.lpr_log2, lpr = 1u << lprl, rpi = 64u >> lprl;
     const uint32_t lir = lane & (lpr - 1), slot = lane >> lprl;
     const uint32_t row0 = wave * rpi * kRows + slot;
@@ -706,11 +711,13 @@ int launch_gated(const GemvArgs &a, uint32_t m, uint32_t groups, hipStream_t s) 
         if (m != MM) return launch_gated<SCHEME, SPL, PAIRS, MM - 1>(a, m, groups, s);
         const uint32_t rows_per_wave = groups * PAIRS;
         const uint32_t waves = (a.n + rows_per_wave - 1) / rows_per_wave;
-        const dim3 grid((waves + waves_for(MM) - 1) / waves_for(MM));
+        constexpr uint32_t kMost = gated_waves_for(SCHEME, MM);
+        const uint32_t wpg = kMost == waves_for(MM) || waves >= 2 * device_simds() ? kMost : waves_for(MM);
+        const dim3 grid((waves + wpg - 1) / wpg);
         if (a.ragged)
-            hipLaunchKernelGGL((gemv_gated_kernel<SCHEME, MM, SPL, PAIRS, true>), grid, dim3(waves_for(MM) * 64), 0, s, a);
+            hipLaunchKernelGGL((gemv_gated_kernel<SCHEME, MM, SPL, PAIRS, true>), grid, dim3(wpg * 64), 0, s, a);
         else
-            hipLaunchKernelGGL((gemv_gated_kernel<SCHEME, MM, SPL, PAIRS, false>), grid, dim3(waves_for(MM) * 64), 0, s, a);
+            hipLaunchKernelGGL((gemv_gated_kernel<SCHEME, MM, SPL, PAIRS, false>), grid, dim3(wpg * 64), 0, s, a);
         return (int)hipGetLastError();
     }
 }

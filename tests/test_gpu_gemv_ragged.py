@@ -127,7 +127,8 @@ def test_many_ragged_rows_take_fewer_lanes(scheme, n, k, swiglu):
     want = O.matmul(scheme, some, len(some), k, x, O.BF16)
     if swiglu:
         g, u = want[:, :len(cols)].astype(np.float64), want[:, len(cols):].astype(np.float64)
-        want = (g / (1.0 + np.exp(-g)) * u).astype(np.float32)
+        with np.errstate(over="ignore"):  # exp(-g) past 1e308: g / inf is the 0 that it stands for
+            want = (g / (1.0 + np.exp(-g)) * u).astype(np.float32)
     whole = ffi.matmul(w, scheme, n, k, xd, w_scales=sc, swiglu=swiglu)
     check_close(whole.cpu().numpy()[:, cols], want, f"{scheme} n={n} k={k}")
     for m in (1, 2, 4, 5):

@@ -121,3 +121,12 @@ def test_gated_streaming_where_it_is_faster(runtime, scheme, k, streams):
     names = kernels(runtime, [("matmul", dict(scheme=scheme, m=m, n=14336, k=k, epilogue=3)) for m in (1, 2, 3, 4, 5)])
     for m, (name,) in zip((1, 2, 3, 4, 5), names):
         assert name.startswith("gemv_gated_stream_kernel" if m in streams else "gemv_gated_kernel"), (m, name)
+
+
+def test_gated_iq3s_workgroups(runtime):
+    """IQ3_S: four waves share the codebook's table where there are two waves a
+    SIMD, one wave a workgroup below (1024 SIMDs); other schemes one from m = 3."""
+    calls = [(ffi.IQ3_S, 2047), (ffi.IQ3_S, 2048), (ffi.Q6_K, 2048)]
+    out = launch_record.record(runtime, [("matmul", dict(scheme=s, m=8, n=n, k=2048, epilogue=3)) for s, n in calls])
+    blocks = [(g[0], b[0]) for _, _, launches in out for _, g, b in launches]
+    assert blocks == [(2047, 64), (512, 256), (2048, 64)]
