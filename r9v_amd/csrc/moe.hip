@@ -1101,29 +1101,28 @@ static uint32_t lpr_for(uint32_t k, uint32_t &nseg) {
     return l2;
 }
 
-int r9vx_moe_sort_stage(const r9vx_moe_problem &p, const MoeLayout &L, hipStream_t s, bool *x16_done) {
+int r9vx_moe_sort_stage(const r9vx_moe_problem &p, const MoeLayout &L, hipStream_t s, bool rows) {
     SortArgs a{p.ids, p.ws, L, p.t * p.k, p.e, p.k, p.t, p.shared};
-    if (x16_done) {
+    if (rows) {
         a.x = p.x;
         a.x16 = reinterpret_cast<_Float16 *>(p.ws + L.x16);
         a.xscale = reinterpret_cast<float *>(p.ws + L.xscale);
         a.dm = p.dm;
         a.xperm = r9vx_group_order(p.scheme_gu);
-        *x16_done = true;
     }
     if (a.p <= 1024) {
         /* sixteen activation rows per further workgroup, beside the sort (a
          * launch of their own took 5.3 us at T = 48) */
-        hipLaunchKernelGGL(sort_small_kernel, dim3(1 + (x16_done ? (a.t + 15) / 16 : 0)), dim3(1024), 0, s, a);
+        hipLaunchKernelGGL(sort_small_kernel, dim3(1 + (rows ? (a.t + 15) / 16 : 0)), dim3(1024), 0, s, a);
         return (int)hipGetLastError();
     }
     const uint32_t nchunk = (a.p + 255) / 256;
     a.nchunk = nchunk;
-    /* x16_done: the activation rows go with the four kernels, 20 / 20 / 40
+    /* the activation rows go with the four kernels, 20 / 20 / 40
      * / 20 % of them (the one-workgroup finish kernel leaves the most CUs
      * idle), four rows per 256-thread workgroup, sixteen per 1024 */
     uint32_t xr[5] = {0, 0, 0, 0, 0};
-    if (x16_done) {
+    if (rows) {
         constexpr uint32_t kCum[5] = {0, 20, 40, 80, 100};
         for (int i = 1; i <= 4; ++i) xr[i] = (uint32_t)((uint64_t)p.t * kCum[i] / 100);
     }

@@ -820,9 +820,8 @@ int r9vx_launch_moe(const r9vx_moe_problem &p, hipStream_t s) {
     if (r9vx_moe_decode_form(p)) { /* pair-order rows: no sort; the combine checks the ids */
         rc = r9vx_moe_decode_stage(p, L, s);
     } else {
-        bool x16_done = false;
-        rc = r9vx_moe_sort_stage(p, L, s, &x16_done);
-        if (!rc) rc = r9vx_moe_grouped_stage(p, L, s, x16_done);
+        rc = r9vx_moe_sort_stage(p, L, s, true);
+        if (!rc) rc = r9vx_moe_grouped_part(p, L, 0, s);
     }
     if (rc) return rc;
     return r9vx_moe_combine_stage(p, L, s);
@@ -831,7 +830,7 @@ int r9vx_launch_moe(const r9vx_moe_problem &p, hipStream_t s) {
 int r9vx_launch_moe_sort(const r9vx_moe_problem &p, uint32_t *counts, uint32_t *offsets, uint32_t *sorted,
                          hipStream_t s) {
     MoeLayout L = r9vx_moe_layout(p.t_bucket, p.e, p.k, p.dm, p.dff, p.shared);
-    int rc = r9vx_moe_sort_stage(p, L, s);
+    int rc = r9vx_moe_sort_stage(p, L, s, false);
     if (rc) return rc;
     uint64_t pp = (uint64_t)p.t * p.k;
     rc = (int)hipMemcpyAsync(counts, p.ws + L.counts, 4ull * p.e, hipMemcpyDeviceToDevice, s);

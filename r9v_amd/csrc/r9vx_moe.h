@@ -102,13 +102,12 @@ struct MoeCombineArgs {
  * whatever the launch's t. */
 inline bool r9vx_moe_decode_form(const r9vx_moe_problem &p) { return p.t_bucket <= 8; }
 
-/* x16_done != NULL: the sort kernels also convert the activation rows for
- * the grouped GEMMs (*x16_done says so). */
-int r9vx_moe_sort_stage(const r9vx_moe_problem &p, const MoeLayout &L, hipStream_t s, bool *x16_done = nullptr);
+/* rows: the sort kernels also convert the activation rows for the grouped GEMMs. */
+int r9vx_moe_sort_stage(const r9vx_moe_problem &p, const MoeLayout &L, hipStream_t s, bool rows);
 int r9vx_moe_decode_stage(const r9vx_moe_problem &p, const MoeLayout &L, hipStream_t s);
-int r9vx_moe_grouped_stage(const r9vx_moe_problem &p, const MoeLayout &L, hipStream_t s, bool x16_done = false);
-int r9vx_moe_grouped_part(const r9vx_moe_problem &p, const MoeLayout &L, uint32_t part, hipStream_t s,
-                          bool x16_done = false);
+/* part 0: the whole grouped stage, on rows the sort has converted; 1: the gate/up
+ * GEMM only; 2: the down GEMM only (1 and 2 on a workspace the whole stage has filled). */
+int r9vx_moe_grouped_part(const r9vx_moe_problem &p, const MoeLayout &L, uint32_t part, hipStream_t s);
 int r9vx_moe_combine_stage(const r9vx_moe_problem &p, const MoeLayout &L, hipStream_t s);
 
 /* Byte offset (from L.o) of the grouped path's per-(row, 64-column) scales. */
