@@ -42,3 +42,12 @@ def test_guard_parser_flags_a_spill():
     res = B.parse_resources(text)
     assert list(res.values())[0]["vgpr_spill"] == 2
     assert len(B.spill_problems(res)) == 1
+
+
+@pytest.mark.parametrize("kernel", ["gemm_thin_kernelILi3ELi8ELi2E", "gemv_gated_stream_kernelILi11ELi4ELi2ELb0E"])
+def test_guard_covers_kernels_at_their_register_limit(kernel):
+    text = (f"x.hip:1:1: remark: Function Name: _ZN12_GLOBAL__N_116{kernel}EEvNS_8ThinArgsE "
+            "[-Rpass-analysis=kernel-resource-usage]\n"
+            "x.hip:1:1: remark:     VGPRs: 128 [-Rpass-analysis=kernel-resource-usage]\n"
+            "x.hip:1:1: remark:     VGPRs Spill: 1 [-Rpass-analysis=kernel-resource-usage]\n")
+    assert len(B.spill_problems(B.parse_resources(text))) == 1
