@@ -45,12 +45,13 @@ int r9vx_probe_expf_check_launch(uint32_t first_bits, uint32_t n, const float *w
 int r9vx_probe_moe_stage_launch(const r9vx_moe_ffn_static *st, const r9vx_moe_ffn_args *args, uint32_t stage,
                                 r9vx_stream_t stream);
 
-/* r9vx_matmul_launch (bf16 activations, m_bucket > 8) on the thin tiles of nr x
- * 32 rows by nc x 32 columns a workgroup, whatever kernel the sizes would
- * choose, so that each shape can be run and timed at any size.  The outputs are
- * the bits of r9vx_matmul_launch's.  A shape that does not exist is refused. */
-int r9vx_probe_matmul_thin_launch(const r9vx_matmul_static *st, const r9vx_matmul_args *args, uint32_t nr, uint32_t nc,
-                                  r9vx_stream_t stream);
+/* r9vx_matmul_launch (bf16 activations, m_bucket > 8) on a named prefill kernel,
+ * whatever the sizes would choose, so that each can be run and timed at any
+ * size: the thin tiles of nr x 32 rows by nc x 32 columns a workgroup, or with
+ * nr = nc = 0 the 256 x 256 tiles.  The outputs are the bits of
+ * r9vx_matmul_launch's.  A shape that does not exist is refused. */
+int r9vx_probe_matmul_tiles_launch(const r9vx_matmul_static *st, const r9vx_matmul_args *args, uint32_t nr,
+                                   uint32_t nc, r9vx_stream_t stream);
 
 #ifdef __cplusplus
 }

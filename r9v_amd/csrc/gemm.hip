@@ -360,7 +360,8 @@ int r9vx_launch_x_to_f16(const uint16_t *x, uint32_t m, uint32_t k, _Float16 *x1
     return (int)hipGetLastError();
 }
 
-int r9vx_launch_gemm(const r9vx_gemm_problem &p, hipStream_t stream) {
+/* The problem with its whole rows (plan_chunks cuts them). */
+static GemmArgs gemm_args(const r9vx_gemm_problem &p) {
     _Float16 *x16 = reinterpret_cast<_Float16 *>(p.workspace);
     float *scale = reinterpret_cast<float *>(reinterpret_cast<uint8_t *>(p.workspace) + r9vx_gemm_x16_bytes(p.m, p.k));
     GemmArgs a{};
@@ -383,23 +384,33 @@ int r9vx_launch_gemm(const r9vx_gemm_problem &p, hipStream_t stream) {
     a.k = p.k;
     a.y_bf16 = p.y_dtype == R9VX_DTYPE_BF16;
     a.epilogue = p.epilogue;
-    /* Two kernels for every scheme and shape, chosen by size: gemm3_kernel
-     * (256 x 256 tiles) and the thin tiles of gemm_thin.hip.  Both give each
-     * output element the same arithmetic -- the K order of the MFMA slices,
-     * how a weight is rounded to fp16 -- which follows from the scheme and k
-     * alone, never from the launch's row count: a row's outputs are the same
-     * bits whatever rows share the launch, at whatever index, and in every
-     * bucket above the decode GEMV's.  The A copies address x16 with 32-bit
-     * offsets, so rows go in launches of at most 2^31 / k elements' worth
-     * (which rows share a launch changes no bit either). */
+    return a;
+}
+
+/* Two kernels for every scheme and shape, chosen by size: gemm3_kernel
+ * (256 x 256 tiles) and the thin tiles of gemm_thin.hip.  Both give each
+ * output element the same arithmetic -- the K order of the MFMA slices,
+ * how a weight is rounded to fp16 -- which follows from the scheme and k
+ * alone, never from the launch's row count: a row's outputs are the same
+ * bits whatever rows share the launch, at whatever index, and in every
+ * bucket above the decode GEMV's. */
+int r9vx_launch_gemm(const r9vx_gemm_problem &p, hipStream_t stream) {
     const uint32_t cus = r9vx_device_cus();
-    {
-        GemmArgs whole = a;
-        const uint32_t wgs = plan_chunks(whole, cus);
-        uint32_t nr = 0, nc = 0;
-        if (thin_plan(p.m, p.n, p.k, p.scheme, cus, nr, nc) < gemm3_cost(whole, p.scheme, wgs, cus))
-            return r9vx_launch_gemm_thin(p, nr, nc, stream);
-    }
+    GemmArgs a = gemm_args(p);
+    const uint32_t wgs = plan_chunks(a, cus);
+    uint32_t nr = 0, nc = 0;
+    if (thin_plan(p.m, p.n, p.k, p.scheme, cus, nr, nc) < gemm3_cost(a, p.scheme, wgs, cus))
+        return r9vx_launch_gemm_thin(p, nr, nc, stream);
+    return r9vx_launch_gemm3(p, stream);
+}
+
+/* The A copies address x16 with 32-bit offsets, so rows go in launches of at
+ * most 2^31 / k elements' worth (which rows share a launch changes no bit). */
+int r9vx_launch_gemm3(const r9vx_gemm_problem &p, hipStream_t stream) {
+    const uint32_t cus = r9vx_device_cus();
+    const GemmArgs a = gemm_args(p);
+    _Float16 *const x16 = const_cast<_Float16 *>(a.x16);
+    float *const scale = const_cast<float *>(a.scale);
     const int rc = r9vx_launch_x_to_f16(p.x, p.m, p.k, x16, scale, r9vx_group_order(p.scheme), stream);
     if (rc) return rc;
     const uint32_t max_rows = (uint32_t)(((1ull << 31) - 1) / p.k) & ~31u;

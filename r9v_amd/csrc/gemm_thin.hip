@@ -355,6 +355,7 @@ void launch_x16(uint32_t order, const uint16_t *x, uint32_t m, uint32_t k, _Floa
 }  // namespace
 
 int r9vx_launch_gemm_thin(const r9vx_gemm_problem &p, uint32_t nr, uint32_t nc, hipStream_t stream) {
+    if (nr == 0 || nc == 0) return (int)hipErrorInvalidValue;
     ThinArgs a{};
     _Float16 *x16 = reinterpret_cast<_Float16 *>(p.workspace);
     float *scale = reinterpret_cast<float *>(reinterpret_cast<uint8_t *>(p.workspace) +

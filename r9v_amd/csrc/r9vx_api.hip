@@ -175,17 +175,17 @@ uint64_t r9vx_matmul_static_flops(const r9vx_matmul_static *st, uint32_t m) {
     return (st->epilogue == R9VX_EPILOGUE_SWIGLU ? 4ull : 2ull) * m * st->n * st->k;
 }
 
-/* nr, nc: the thin tiles' shape (0, 0: the kernel by the size rule) */
-static int matmul_launch(const char *op, const r9vx_matmul_static *st, const r9vx_matmul_args *a, uint32_t nr,
-                         uint32_t nc, r9vx_stream_t stream) {
+/* tiles: the prefill kernel, a probe's {nr, nc} (NULL: by the size rule) */
+static int matmul_launch(const char *op, const r9vx_matmul_static *st, const r9vx_matmul_args *a,
+                         const uint32_t (*tiles)[2], r9vx_stream_t stream) {
     Problems pr;
     if (!st || !a) {
         pr.add(R9VX_ERR_NULL, "static and args must be non-NULL");
         return pr.finish(op);
     }
     check_matmul_static(st, pr);
-    if (nr && (st->in_dtype != R9VX_DTYPE_BF16 || st->m_bucket <= 8))
-        pr.add(R9VX_ERR_UNSUPPORTED, "the thin tiles take bf16 activations and m_bucket > 8");
+    if (tiles && (st->in_dtype != R9VX_DTYPE_BF16 || st->m_bucket <= 8))
+        pr.add(R9VX_ERR_UNSUPPORTED, "the prefill kernels take bf16 activations and m_bucket > 8");
     if (a->m > st->m_bucket)
         pr.add(R9VX_ERR_INVALID, "m=%u exceeds m_bucket=%u", a->m, st->m_bucket);
     if (a->m > 0) {
@@ -242,7 +242,9 @@ static int matmul_launch(const char *op, const r9vx_matmul_static *st, const r9v
         g.scheme = st->w_scheme;
         g.y_dtype = st->out_dtype;
         g.epilogue = st->epilogue;
-        return hip_status(op, nr ? r9vx_launch_gemm_thin(g, nr, nc, s) : r9vx_launch_gemm(g, s));
+        if (!tiles) return hip_status(op, r9vx_launch_gemm(g, s));
+        const uint32_t nr = (*tiles)[0], nc = (*tiles)[1];
+        return hip_status(op, nr || nc ? r9vx_launch_gemm_thin(g, nr, nc, s) : r9vx_launch_gemm3(g, s));
     }
     /* GEMV, eight activation rows per launch. */
     const uint32_t xe = st->in_dtype == R9VX_DTYPE_F32 ? 4 : 2;
@@ -271,17 +273,13 @@ static int matmul_launch(const char *op, const r9vx_matmul_static *st, const r9v
 }
 
 int r9vx_matmul_launch(const r9vx_matmul_static *st, const r9vx_matmul_args *a, r9vx_stream_t stream) {
-    return matmul_launch("matmul", st, a, 0, 0, stream);
+    return matmul_launch("matmul", st, a, nullptr, stream);
 }
 
-int r9vx_probe_matmul_thin_launch(const r9vx_matmul_static *st, const r9vx_matmul_args *a, uint32_t nr, uint32_t nc,
-                                  r9vx_stream_t stream) {
-    if (nr == 0 || nc == 0) {
-        Problems pr;
-        pr.add(R9VX_ERR_INVALID, "nr=%u, nc=%u: no thin tile is empty", nr, nc);
-        return pr.finish("probe_matmul_thin");
-    }
-    return matmul_launch("probe_matmul_thin", st, a, nr, nc, stream);
+int r9vx_probe_matmul_tiles_launch(const r9vx_matmul_static *st, const r9vx_matmul_args *a, uint32_t nr, uint32_t nc,
+                                   r9vx_stream_t stream) {
+    const uint32_t tiles[2] = {nr, nc};
+    return matmul_launch("probe_matmul_tiles", st, a, &tiles, stream);
 }
 
 /* ----------------------------------------------------------- weights/decode */

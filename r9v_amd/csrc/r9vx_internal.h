@@ -116,6 +116,8 @@ size_t r9vx_gemm_workspace_bytes(uint32_t m_bucket, uint32_t k);
 /* Bytes of the fp16 rows in it; the row scales follow. */
 size_t r9vx_gemm_x16_bytes(uint32_t m, uint32_t k);
 int r9vx_launch_gemm(const r9vx_gemm_problem &p, hipStream_t stream);
+/* On the 256-column tiles whatever the sizes. */
+int r9vx_launch_gemm3(const r9vx_gemm_problem &p, hipStream_t stream);
 /* The thin-tile form (gemm_thin.hip): nr row tiles of 32 rows and nc column
  * tiles of 32 columns per workgroup.  Output bits equal r9vx_launch_gemm's.
  * Shapes that do not exist are refused.  They are (nr, nc, ns, load): the last

@@ -122,7 +122,7 @@ EXPORTS = [
     ("r9vx_probe_stream_blocks", [ctypes.c_uint64], _U32),
     ("r9vx_probe_mfma_launch", [_U32, _U32, _P, _P], ctypes.c_int),
     ("r9vx_probe_moe_stage_launch", [_P, _P, _U32, _P], ctypes.c_int),
-    ("r9vx_probe_matmul_thin_launch", [_P, _P, _U32, _U32, _P], ctypes.c_int),
+    ("r9vx_probe_matmul_tiles_launch", [_P, _P, _U32, _U32, _P], ctypes.c_int),
     ("r9vx_probe_expf_check_launch", [_U32, _U32, _P, _P, _P], ctypes.c_int),
     # include/r9vx_gguf.h
     ("r9vx_gguf_parse", [_P, _U64, _P], ctypes.c_int),
@@ -496,10 +496,11 @@ def probe_mfma(blocks, iters, sink=None, stream=None):
     return sink
 
 
-def probe_matmul_thin(w, w_scheme, n, k, x, nr, nc, out_dtype=F32, bias=None, residual=None, w_scales=None,
-                      stream=None):
+def probe_matmul_tiles(w, w_scheme, n, k, x, nr, nc, out_dtype=F32, bias=None, residual=None, w_scales=None,
+                       stream=None):
     """matmul (bf16 x, its rows' bucket above 8) on the thin tiles of nr x 32
-    rows by nc x 32 columns, whatever kernel the sizes would choose."""
+    rows by nc x 32 columns, or with 0, 0 the 256 x 256 tiles, whatever kernel
+    the sizes would choose."""
     torch = _need_gpu(w, x, bias, residual, w_scales)
     m = x.shape[0]
     y = torch.empty((m, n), dtype=torch.float32 if out_dtype == F32 else torch.bfloat16, device=x.device)
@@ -508,7 +509,7 @@ def probe_matmul_thin(w, w_scheme, n, k, x, nr, nc, out_dtype=F32, bias=None, re
     workspace = torch.empty(matmul_workspace_bytes(st), dtype=torch.uint8, device=x.device)
     args = MatmulArgs(_ptr(w), _ptr(w_scales), None, _ptr(x), None, _ptr(bias), _ptr(residual), _ptr(y),
                       _ptr(workspace), m, 0)
-    _check(load().r9vx_probe_matmul_thin_launch(ctypes.byref(st), ctypes.byref(args), nr, nc, _stream(torch, stream)))
+    _check(load().r9vx_probe_matmul_tiles_launch(ctypes.byref(st), ctypes.byref(args), nr, nc, _stream(torch, stream)))
     return y
 
 

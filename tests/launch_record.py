@@ -31,14 +31,14 @@ def launches():
     hip.record_clear()
     return out
 
-def matmul(scheme, m, n, k, m_bucket=None, x_f32=False, bf16_out=False, epilogue=0, thin=None):
+def matmul(scheme, m, n, k, m_bucket=None, x_f32=False, bf16_out=False, epilogue=0, tiles=None):
     st = ffi.matmul_static(n=n, k=k, w_scheme=scheme, in_dtype=ffi.F32 if x_f32 else ffi.BF16,
                            out_dtype=ffi.BF16 if bf16_out else ffi.F32, m_bucket=m_bucket or m, epilogue=epilogue)
     split = scheme in ffi.SPLIT_SCHEMES
     args = ffi.MatmulArgs(FAKE, FAKE if split else None, None, FAKE, None, FAKE if epilogue == 1 else None,
                           FAKE if epilogue == 2 else None, FAKE, FAKE, m, 0)
-    if thin:
-        return L.r9vx_probe_matmul_thin_launch(ctypes.byref(st), ctypes.byref(args), *thin, None)
+    if tiles:
+        return L.r9vx_probe_matmul_tiles_launch(ctypes.byref(st), ctypes.byref(args), *tiles, None)
     return L.r9vx_matmul_launch(ctypes.byref(st), ctypes.byref(args), None)
 
 def route(t, e, k, scoring=0):

@@ -131,7 +131,7 @@ def test_matmul_prefill_bucket_2048_configs2_shape(scheme):
 
 @pytest.mark.parametrize("scheme", [O.Q4_K, O.IQ4_XS])
 def test_matmul_prefill_ragged_n(scheme):
-    """N % 256 != 0 (the register-decoded 256 x 256 tile) at m_bucket 512."""
+    """N % 256 != 0 at m_bucket 512 (thin tiles of every row count's choice)."""
     n, k = 5000, 2048
     w_h = synth.quant_weights(scheme, 8500, n, k)
     runs = [(1, 0, False), (9, 3, False), (300, 299, False), (512, 200, True), (512, 511, False)]
@@ -143,8 +143,8 @@ def test_matmul_prefill_ragged_n(scheme):
 @pytest.mark.parametrize("scheme,n", [(O.Q8_0, 300), (O.Q8_0, 512), (O.Q6_K, 300), (O.Q6_K, 512), (O.IQ3_S, 300),
                                       (O.IQ3_S, 512)])
 def test_matmul_prefill_repacked_schemes(scheme, n):
-    """Q8_0 / Q6_K / IQ3_S at m_bucket 64 on the 256 x 256 loop, with a
-    ragged last weight block (n = 300) and whole blocks (n = 512)."""
+    """Q8_0 / Q6_K / IQ3_S at m_bucket 64 (thin tiles), with a ragged last column
+    tile (n = 300) and whole ones (n = 512)."""
     k = 1024
     wire = synth.quant_weights(scheme, 8600 + scheme + n, n, k)
     w, sc = ffi.repack(dev(wire), scheme, n, k)

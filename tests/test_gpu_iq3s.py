@@ -137,11 +137,11 @@ def test_prefill_gemm_parity(m, n, k):
     check_close(y, O.matmul(IQ3_S, w, n, k, x, O.BF16, threads=8), f"m={m} n={n} k={k}")
 
 
-# m > 8 runs the 256 x 256 loop for every n (two threads per weight row, a
-# thread's half K step one 32-weight group: its 8 grid indices, sign word and
-# the block's side word, decoded through the signed grid table in LDS); these
-# shapes reach its row-chunk plans with ragged row tiles and the bias
-# epilogue.
+# m > 8 on the kernel that the sizes choose (thin tiles or the 256 x 256 loop; in
+# both a thread's half K step is one 32-weight group: its 8 grid indices, sign
+# word and the block's side word, decoded through the signed grid table in LDS),
+# with ragged row tiles and the bias epilogue.  test_gpu_prefill_tiles.py runs
+# these shapes on each by name.
 @pytest.mark.parametrize("m,n,k", [(9, 256, 512), (700, 2560, 512), (1100, 5376, 512), (2048, 4096, 1024)])
 def test_prefill_gemm_256_tile(m, n, k):
     w = synth.quant_weights(IQ3_S, 3400 + m, n, k)

@@ -264,7 +264,8 @@ def test_gemm_large_ragged_shapes(scheme, m, n, k):
 
 
 # Epilogues and bf16 output with n a multiple of 256, with a ragged last
-# block (n % 8 == 0: 16-byte rows), and with n % 8 != 0 (element stores).
+# block (n % 8 == 0: 16-byte rows) on the 256 x 256 tiles, and with n % 8 != 0
+# on thin ones (element stores).
 @pytest.mark.parametrize("n", [28000, 28160, 1001])
 def test_gemm_epilogues_ragged_n(n):
     m, k = 600, 256
@@ -280,10 +281,10 @@ def test_gemm_epilogues_ragged_n(n):
 
 
 # The 256-column GEMM (gemm3_kernel) cuts each weight block's rows into
-# chunks sized to fill whole rounds of the CUs; these shapes reach its plans:
-# one block, one 32-row tile per chunk, every block with the same chunk
-# count (the XCD band order), two chunk counts across blocks, several
-# rounds, ragged last row tiles.
+# chunks sized to fill whole rounds of the CUs; of these shapes the last three
+# reach its plans (every block with the same chunk count in the XCD band order,
+# two chunk counts across blocks, several rounds, ragged last row tiles), the
+# first two are thin tiles' (test_gpu_prefill_tiles.py runs each on both).
 @pytest.mark.parametrize("scheme", [O.Q4_K, O.IQ4_XS])
 @pytest.mark.parametrize("m,n", [(9, 256), (700, 2560), (2048, 4096), (1100, 5376), (2600, 14336)])
 def test_gemm_row_chunk_plans(scheme, m, n):
@@ -351,8 +352,8 @@ def test_gemm_row_permutation_invariance_full_size():
 
 @pytest.mark.parametrize("m,n,k", [(16, 64, 512), (520, 32768, 256)])
 def test_gemm_large_activation_rows_scaled_exactly(m, n, k):
-    """Rows with |x| >= 2^15 go through the power-of-two row scale (the
-    128-row tile and the 256-row LDS-decoded tile)."""
+    """Rows with |x| >= 2^15 go through the power-of-two row scale (the thin
+    tiles and the 256-row tiles)."""
     w = synth.quant_weights(O.Q4_K, 7401, n, k)
     xf = synth.normal_f32(7402, (m, k))
     xf[3] *= 1e6

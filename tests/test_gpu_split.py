@@ -163,8 +163,8 @@ PREFILL = [(9, 320, 2048), (40, 1000, 4096), (300, 512, 2048), (129, 2304, 1024)
 @pytest.mark.parametrize("scheme", SCHEMES)
 @pytest.mark.parametrize("m,n,k", PREFILL)
 def test_prefill_gemm_split_layout_parity(scheme, m, n, k):
-    """m > 8: the MFMA GEMM on the split layout (the 256 x 256 loop; a
-    ragged n repeats row n - 1 in its last weight block)."""
+    """m > 8: the MFMA GEMM on the split layout, at few rows (the thin tiles;
+    test_gpu_prefill_tiles.py names each kernel)."""
     w = synth.quant_weights(scheme, 3000 + m + n, n, k)
     x = synth.normal_bf16(4000 + m + k, (m, k))
     body, scales = ffi.repack(dev(w), scheme, n, k)
@@ -172,12 +172,10 @@ def test_prefill_gemm_split_layout_parity(scheme, m, n, k):
     check_close(y, O.matmul(scheme, w, n, k, x, O.BF16, threads=8), f"scheme={scheme} m={m} n={n} k={k}")
 
 
-# Q8_0 / Q6_K run the 256 x 256 loop (every n) that decodes each
-# weight tile once into LDS (two threads per weight row; a thread's half K
-# step is one Q8_0 block, or 16 Q6_K ql bytes and their 16 qh bytes, loaded
-# two steps ahead); these shapes reach its row-chunk plans (one block,
-# uniform chunks in the XCD band order, two chunk counts, several rounds)
-# with ragged last row tiles and the bias epilogue.
+# Q8_0 / Q6_K on the kernel that the sizes choose (thin tiles or the 256 x 256
+# loop: a thread's half K step there is one Q8_0 block, or 16 Q6_K ql bytes and
+# their 16 qh bytes, loaded two steps ahead), with ragged last row tiles and the
+# bias epilogue.  test_gpu_prefill_tiles.py runs these shapes on each by name.
 @pytest.mark.parametrize("scheme", SCHEMES)
 @pytest.mark.parametrize("m,n,k", [(9, 256, 512), (700, 2560, 512), (1100, 5376, 512), (2048, 4096, 1024)])
 def test_prefill_gemm_split_256_tile(scheme, m, n, k):
@@ -193,8 +191,7 @@ def test_prefill_gemm_split_256_tile(scheme, m, n, k):
 
 @pytest.mark.parametrize("scheme", SCHEMES)
 def test_prefill_gemm_split_large_sampled(scheme):
-    """A 1024 x 4096 x 4096 launch (16 K tiles of rows, 16 column tiles):
-    sampled rows against the oracle, residual epilogue and bf16 output."""
+    """A 1024 x 4096 x 4096 launch (eight-chain thin tiles): sampled rows against the oracle, residual epilogue and bf16 output."""
     m, n, k = 1024, 4096, 4096
     w = synth.quant_weights(scheme, 5151, n, k)
     x = synth.normal_bf16(5152, (m, k))

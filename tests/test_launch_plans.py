@@ -46,7 +46,7 @@ def test_prefill_rows_within_the_launch_limits(runtime, m, n, k):
     tiles every row converted once and in a tile."""
     call = dict(scheme=ffi.Q4_K, m=m, n=n, k=k)
     (rc, msg, _), (thin_rc, thin_msg, launches) = launch_record.record(
-        runtime, [("matmul", call), ("matmul", dict(call, thin=(8, 2)))])
+        runtime, [("matmul", call), ("matmul", dict(call, tiles=(8, 2)))])
     assert rc == 0, msg
     assert thin_rc == 0, thin_msg
     thin = [(name, g) for name, g, _ in launches if name.startswith("gemm_thin_kernel")]
@@ -63,15 +63,15 @@ THIN_SHAPES = [(1, 1), (2, 1), (4, 1), (1, 2), (2, 2), (4, 2), (8, 2)]
 def test_thin_shapes_launch_or_are_refused(runtime, scheme):
     """Every pair of row and column tiles runs its kernel or is an error: none
     returns 0 with nothing launched."""
-    pairs = [(nr, nc) for nr in (1, 2, 3, 4, 6, 8, 16) for nc in (1, 2, 4)]
-    out = launch_record.record(runtime, [("matmul", dict(scheme=scheme, m=300, n=500, k=512, thin=p)) for p in pairs])
+    pairs = [(nr, nc) for nr in (1, 2, 3, 4, 6, 8, 16) for nc in (1, 2, 4)] + [(0, 1), (2, 0)]
+    out = launch_record.record(runtime, [("matmul", dict(scheme=scheme, m=300, n=500, k=512, tiles=p)) for p in pairs])
     for (nr, nc), (rc, _, launches) in zip(pairs, out):
         ran = [k for k, _, _ in launches if k.startswith("gemm")]
         assert ran == ([f"gemm_thin_kernel<{scheme}, {nr}, {nc}>"] if (nr, nc) in THIN_SHAPES else []), (nr, nc)
         assert (rc == 0) == bool(ran), (nr, nc, rc)
     # and the decode bucket and f32 activations have none
     for kw in (dict(m=8), dict(m=300, x_f32=True), dict(m=300, scheme=ffi.Q4_K, x_f32=True)):
-        call = dict(dict(scheme=scheme, n=500, k=512, thin=(1, 1)), **kw)
+        call = dict(dict(scheme=scheme, n=500, k=512, tiles=(1, 1)), **kw)
         assert launch_record.record(runtime, [("matmul", call)])[0][0] < 0
 
 
@@ -130,3 +130,18 @@ def test_gated_iq3s_workgroups(runtime):
     out = launch_record.record(runtime, [("matmul", dict(scheme=s, m=8, n=n, k=2048, epilogue=3)) for s, n in calls])
     blocks = [(g[0], b[0]) for _, _, launches in out for _, g, b in launches]
     assert blocks == [(2047, 64), (512, 256), (2048, 64)]
+
+
+# kernels that the GPU tests' texts name for their sizes, all schemes
+NAMED = [(3000, 8481, 768, "gemm3_kernel"), (300, 8481, 768, "gemm_thin_kernel 4, 2"), (64, 8481, 768, "gemm_thin_kernel 2, 2"),
+         (9, 8481, 768, "gemm_thin_kernel 1, 2"), (1024, 4096, 4096, "gemm_thin_kernel 8, 2"),
+         (129, 257, 2048, "gemm_thin_kernel 1, 1"), (2600, 14336, 512, "gemm3_kernel"), (520, 32768, 256, "gemm3_kernel"),
+         (600, 28000, 256, "gemm3_kernel"), (600, 1001, 256, "gemm_thin_kernel 4, 1")]
+
+
+@pytest.mark.parametrize("scheme", [ffi.Q4_K, ffi.IQ4_XS, ffi.Q6_K, ffi.Q8_0, ffi.IQ3_S])
+def test_kernels_named_by_the_gpu_tests(runtime, scheme):
+    names = kernels(runtime, [("matmul", dict(scheme=scheme, m=m, n=n, k=k)) for m, n, k, _ in NAMED])
+    for (m, n, k, want), ran in zip(NAMED, names):
+        kernel, _, shape = want.partition(" ")
+        assert ran[-1] == f"{kernel}<{scheme}{', ' + shape if shape else ''}>", (m, n, k)
