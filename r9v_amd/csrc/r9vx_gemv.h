@@ -416,9 +416,10 @@ int launch_stream(const GemvArgs &a, uint32_t simds, hipStream_t s) {
  * that receives a row's gate sum also holds its up sum.  bf16 activations,
  * general lane mapping (runtime lanes per row and K segments).  PAIRS gate/up
  * row pairs per lane group: the launcher takes two when n >= 8 x SIMDs and
- * one below (measured, Q4_K, graph replay: n = 14336, K = 4096, M = 4:
- * 39.2 us at two against 49.1 at one and 64.9 at three; n = 2816, K = 2048,
- * M = 8: 11.5 us at one against 21.3 at two). */
+ * one below, for the calls that the streaming form does not take (Q4_K, graph
+ * replay, us at one / two: n = 14336, K = 4096, M = 8 74.5 / 59.7, K = 8192, M = 3
+ * 68.1 / 59.5, M = 5 83.1 / 71.8; n = 2816, K = 2048, M = 8 11.8 / 22.3.  At M = 5
+ * and 6 with K up to 4096 one is the better at this n too: 43.0 / 48.6). */
 /* Waves of a workgroup, at most: IQ3_S rows share the codebook's table (4 KiB to
  * build) between four from 2 x SIMDs waves on (m = 8, n = 16384, K = 1792 55.6 ->
  * 45.1 us; n = 768, K = 512 6.1 / 5.3, so not below). */

@@ -76,14 +76,6 @@ __device__ __forceinline__ void thin_load(const uint8_t *base, uint32_t off, con
     }
 }
 
-/* (a & m) | o with both masks in scalar registers: one instruction where the
- * compiler, with literals, takes two. */
-__device__ __forceinline__ uint32_t thin_and_or_ss(uint32_t a, uint32_t m, uint32_t o) {
-    uint32_t r;
-    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "s"(m), "v"(o));
-    return r;
-}
-
 /* {fp16(dl a + c), fp16(dl b + c)} of one half of each of a, b (fp16 pairs;
  * HI: the high halves), each fused and rounded once. */
 template <bool HI>
@@ -121,8 +113,8 @@ __device__ __forceinline__ void thin_decode(const ThinUnit<SCHEME> &t, uint32_t 
         const uint32_t k1024 = 0x64006400u;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            const uint32_t l02 = thin_and_or_ss(dw[q], 0x000F000Fu, k1024), l13 = thin_and_or_ss(dw[q] >> 8, 0x000F000Fu, k1024);
-            const uint32_t h02 = thin_and_or_ss(dw[q] >> 4, 0x000F000Fu, k1024), h13 = thin_and_or_ss(dw[q] >> 12, 0x000F000Fu, k1024);
+            const uint32_t l02 = r9vx_and_or(dw[q], 0x000F000Fu, k1024), l13 = r9vx_and_or(dw[q] >> 8, 0x000F000Fu, k1024);
+            const uint32_t h02 = r9vx_and_or(dw[q] >> 4, 0x000F000Fu, k1024), h13 = r9vx_and_or(dw[q] >> 12, 0x000F000Fu, k1024);
             dst[64 * q] = r9vx_u32x4{thin_mix<false>(dl0, l02, l13, c0), thin_mix<true>(dl0, l02, l13, c0),
                                      thin_mix<false>(dl1, h02, h13, c1), thin_mix<true>(dl1, h02, h13, c1)};
             if (q == 1) mid();
