@@ -814,7 +814,8 @@ int launch_one(const GemvArgs &a, uint32_t m, uint32_t rows_per_slot_group, hipS
         if constexpr (!XF32) {
             /* several K segments of 64 lanes (K > 4096, or K > 2048 at
              * M >= 5): the same compile-time form with the segment count
-             * read at run time */
+             * read at run time (full rows with an epilogue or bf16 outputs
+             * have no instance of it and take the general form) */
             if (a.lpr_log2 == 6 && a.nseg > 1 && (a.ragged || (a.epilogue == R9VX_EPILOGUE_NONE && !a.y_bf16))) {
                 const uint32_t simds = device_simds();
                 switch (MM <= 2 && a.n < 8 * simds ? 2u : balanced_rows(a.n, simds, MM >= 3 ? 1u : 0u)) {
