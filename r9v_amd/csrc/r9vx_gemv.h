@@ -598,7 +598,10 @@ __global__ __launch_bounds__(256) void gemv_gated_stream_kernel(GemvArgs a, uint
     for (int s = 0; s < SPL; ++s) {
         const uint32_t ci = (uint32_t)s * 64u + lane;
         live[s] = !RAG || ci < a.cpr;
-        cis[s] = live[s] ? ci : a.cpr - 1;
+        /* (clamped for full Q4_K rows too up to m = 3, where the compiler's schedule
+         * without it is 1.4% slower at m = 3; elsewhere it is up to 18% faster) */
+        const bool clamp = RAG || (SCHEME == R9VX_SCHEME_Q4_K && M <= 3);
+        cis[s] = !clamp || ci < a.cpr ? ci : a.cpr - 1;
         uint32_t klo, khi;
         chunk_k<SCHEME>(cis[s], klo, khi);
 #pragma unroll
